@@ -48,8 +48,9 @@ extern "C" {
 #define MLX_E_HIP       206  /* HIP runtime failure                        */
 
 /* precision of the Legendre contractions (trans and vec2tp) */
-#define MLX_PREC_FP64   0    /* FP64 operands, FP64 accumulation (vector
-                                FMA), every column computed: the plain path */
+#define MLX_PREC_FP64   0    /* FP64 operands, FP64 accumulation: FP64 MFMA
+                                where the kit's radial size has MFMA kernels
+                                and no radial offset is set, vector FMA else */
 #define MLX_PREC_FP32   1    /* FP32 operands, FP32 MFMA accumulation       */
 #define MLX_PREC_BF16X3 2    /* 3-term split-BF16 on MFMA: each FP32-staged
                                 operand split into three BF16 terms, six
@@ -133,8 +134,8 @@ int mlx_kit_get(mlx_ctx* ctx, const char* which, double* host, int64_t n);
 
 /* Legendre-contraction precision used by mlx_trans and mlx_vec2tp:
  * MLX_PREC_FP64, MLX_PREC_FP32, MLX_PREC_FP64_MFMA or MLX_PREC_BF16X3.
- * Every precision but MLX_PREC_FP64 runs the MFMA kernels, and the vortex
- * step then skips the modes de-aliasing zeroes. */
+ * Where the kit's radial size has MFMA kernels, every precision runs them,
+ * and the vortex step then skips the modes de-aliasing zeroes. */
 int mlx_set_precision(mlx_ctx* ctx, int prec);
 /* Precision of one contraction site (MLX_STAGE_*) apart from the context's;
  * prec = -1 makes the site follow mlx_set_precision again.  No counterpart

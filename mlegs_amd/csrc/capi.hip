@@ -97,8 +97,7 @@ void trans(mlx_ctx *c, mlx_field *f, const char *space, int rscale = 0) {
         set_space(f, "PFP");
       }
       if (cur == 1) {
-        k_ln_column(c, f->e, f->sc, -1.0);
-        leg_forward(c, f->e, c->scr[0], f->off[0]);
+        leg_forward(c, f->e, c->scr[0], f->off[0], true, -1, true, f->sc);
         swap_scr(c, f);
         set_space(f, "FFP");
       }
@@ -125,9 +124,8 @@ void trans(mlx_ctx *c, mlx_field *f, const char *space, int rscale = 0) {
         set_space(f, "FFP");
       }
       if (cur == 2) {
-        leg_backward(c, f->e, c->scr[0], f->off[0]);
+        leg_backward(c, f->e, c->scr[0], f->off[0], true, -1, true, f->sc);
         swap_scr(c, f);
-        k_ln_column(c, f->e, f->sc, +1.0);
         set_space(f, "PFP");
       }
       if (cur == 1) {
@@ -378,10 +376,7 @@ void febe(mlx_ctx *c, mlx_field *s, const mlx_field *nl, double dt) {
 DealiasLimits dealias_limits(mlx_ctx *c) {
   const KitDev &k = c->kit;
   DealiasLimits d;
-  // the FP64 contraction kernels compute every column and slice: the
-  // restrictions hold only when every site of the advection term runs on MFMA
-  for (int s = 0; s < MLX_STAGE_COUNT; ++s)
-    if (stage_precision(c, s) == MLX_PREC_FP64) return d;
+  // the general contraction kernels compute every column and slice
   if (!mfma_ok(k, 0) || k.np <= 1) return d;
   d.on = true;
   d.pcut = k.np / 3 + 1 > 1 ? k.np / 3 + 1 : 1;
@@ -392,6 +387,13 @@ DealiasLimits dealias_limits(mlx_ctx *c) {
     d.zhi = k.nz - zcut;  // zupper - 2 with zupper = nz - zcut + 2
   }
   return d;
+}
+
+// vec2tp's result is solved over the rows of chi's own radial offset.  The
+// MFMA projection forms the rows below nrchop - m only, so an FP64 result with
+// an offset takes the general projection, which forms the three rows past them.
+bool general_projection(const mlx_ctx *c, const mlx_field *chi) {
+  return chi->off[0] != 0 && stage_precision(c, MLX_STAGE_PROJ) == MLX_PREC_FP64;
 }
 
 // abcn (mlegs_scalar_ops.f90:1200-1262); copy_prev = false skips s_p <- s
@@ -483,7 +485,8 @@ bool tp2vec_back(mlx_ctx *c, mlx_field *ur, mlx_field *up, mlx_field *uz, int nc
   // physical rows only, on the MFMA path: the radial transform hands the
   // phi transform its FP32 even/odd sums (half the bytes of the FP64 rows,
   // which the phi transform forms from them exactly)
-  const bool pairs = lean && phys_rows && (c->prec == MLX_PREC_FP32 || c->prec == MLX_PREC_BF16X3) && mfma_ok(k, 0);
+  const bool pairs = lean && phys_rows && (c->prec == MLX_PREC_FP32 || c->prec == MLX_PREC_BF16X3) && mfma_ok(k, 0) &&
+                     mfma_small(k);
   // the de-aliased kappa slices zlo..zhi of the input are zero
   mlx_field *const three[3] = {ur, up, uz};
   if (!z_done) tp2vec_back_z(c, three, 3, ncols, zlo, zhi);
@@ -987,9 +990,8 @@ void vec2tp_pfp(mlx_ctx *c, mlx_field *ur, mlx_field *up, mlx_field *uz, mlx_fie
   // nothing below (the z transforms, the radial transforms and the
   // projection take columns m < nc, calcat and the log step column 0), so
   // the radial transforms leave them unwritten.
-  k_ln_column(c, up->e, up->sc, -1.0);
   PrecScope ps_up(c, MLX_STAGE_UP);
-  leg_forward(c, up->e, c->scr[0], up->off[0], true, nc, !dl.on);
+  leg_forward(c, up->e, c->scr[0], up->off[0], true, nc, !dl.on, up->sc);
   swap_scr(c, up);
   if (k.nz > 1)
     fft_z(c, up->e, -1, active_pairs(k, up->off[0], nc), k.nrchop + up->off[0], nc, 1, 0, zlo, zhi);
@@ -1002,7 +1004,7 @@ void vec2tp_pfp(mlx_ctx *c, mlx_field *ur, mlx_field *up, mlx_field *uz, mlx_fie
   {
     const int prec_m0 = stage_precision(c, MLX_STAGE_PROJ0);
     PrecScope ps_proj(c, MLX_STAGE_PROJ);
-    vec2tp_project(c, ur->e, up->e, uz->e, psi->e, chi->e, 3, nc, zlo, zhi, prec_m0);
+    vec2tp_project(c, ur->e, up->e, uz->e, psi->e, chi->e, 3, nc, zlo, zhi, prec_m0, general_projection(c, chi));
   }
   set_space(psi, "FFF");
   set_space(chi, "FFF");
@@ -1062,7 +1064,7 @@ int advection_rhs(mlx_ctx *c, mlx_field *psi, mlx_field *chi, mlx_field *nlpsi, 
   mlx_field *wr = tmp(c, 7), *wp = tmp(c, 8), *wz = tmp(c, 9);
   // psi and chi are de-aliased here and so is the result: the MFMA path
   // skips the columns and slices de-aliasing zeroes
-  const DealiasLimits dl = dealias_limits(c);
+  const DealiasLimits dl = general_projection(c, nlchi) ? DealiasLimits() : dealias_limits(c);
   bool f32phys = false;
   {
     // tp2vec and tp2curlvec: both front passes in one launch, then the six

@@ -17,6 +17,13 @@
 // vec2tp (vector_projection, :1387-1436): five parity-folded contractions
 // per (m, k) against the precomputed V, D, T tables, combined in the
 // epilogue into psi and chi.
+//
+// These are the general kernels: any radial size, any radial chopping offset.
+// Every precision, FP64 included, takes the MFMA kernels of legendre_mfma.hip
+// and legendre_f64.hip where mfma_ok holds (same results bit for bit): at 256^3
+// the FP64 forward and backward contractions take 229 and 194 us here against
+// 122 and 106 us there, the projection 756 against 311 us with the de-aliasing
+// limits, and the default FP64 vortex step took 4.36 ms against 2.15.
 #include "mlx_internal.h"
 
 namespace {
@@ -316,13 +323,15 @@ const WorkTable &get_work(mlx_ctx *c, int kind, int nroff) {
 
 namespace mlx {
 
-void leg_forward(mlx_ctx *c, const double2 *in, double2 *out, int nroff, bool zero, int ncols, bool ztail) {
+void leg_forward(mlx_ctx *c, double2 *in, double2 *out, int nroff, bool zero, int ncols, bool ztail,
+                 const double *ln) {
   const KitDev &k = c->kit;
   if (k.nrchop + nroff > k.nrdim_ref) MLX_THROW(MLX_E_ARG, "rtrans_forward: chopping in r too large");
-  if (c->prec != MLX_PREC_FP64 && mfma_ok(k, nroff)) {
-    leg_forward_mfma(c, in, out, ncols, ztail);
+  if (mfma_ok(k, nroff)) {
+    leg_forward_mfma(c, in, out, ncols, ztail, ln);
     return;
   }
+  if (ln) k_ln_column(c, in, ln, -1.0);
   if (zero) HIPCHK(hipMemsetAsync(out, 0, sizeof(double2) * c->nelem, c->stream));
   const WorkTable &wt = get_work(c, 0, nroff);
   if (wt.n == 0) return;
@@ -333,29 +342,34 @@ void leg_forward(mlx_ctx *c, const double2 *in, double2 *out, int nroff, bool ze
   HIPCHK(hipGetLastError());
 }
 
-void leg_backward(mlx_ctx *c, const double2 *in, double2 *out, int nroff, bool zero, int ncols, bool ztail) {
+void leg_backward(mlx_ctx *c, const double2 *in, double2 *out, int nroff, bool zero, int ncols, bool ztail,
+                  const double *ln) {
   const KitDev &k = c->kit;
   if (k.nrchop + nroff > k.nrdim_ref) MLX_THROW(MLX_E_ARG, "rtrans_backward: chopping in r too large");
-  if (c->prec != MLX_PREC_FP64 && mfma_ok(k, nroff)) {
-    leg_backward_mfma(c, in, out, ncols, ztail);
+  if (mfma_ok(k, nroff)) {
+    leg_backward_mfma(c, in, out, ncols, ztail, ln);
     return;
   }
   if (zero) HIPCHK(hipMemsetAsync(out, 0, sizeof(double2) * c->nelem, c->stream));
   const WorkTable &wt = get_work(c, 1, nroff);
-  if (wt.n == 0) return;
+  if (wt.n == 0) {
+    if (ln) k_ln_column(c, out, ln, +1.0);
+    return;
+  }
   dim3 grid(wt.n, (k.nzdim + BN - 1) / BN);
   ProbeScope probe(c, MLX_PROBE_LEG_BWD, leg_bytes(k, nroff, 8), leg_flops(k, nroff));
   probed_launch(probe, k_leg_bwd_f64, grid, dim3(256), 0, c->stream, in, out, k.pf, wt.d, k.nrdim, k.npdim, k.nzdim,
                      k.nr, k.nrh, k.ne);
   HIPCHK(hipGetLastError());
+  if (ln) k_ln_column(c, out, ln, +1.0);
 }
 
-// ncols, zlo, zhi: as vec2tp_project_f32 on the MFMA path; the FP64 path
-// computes every column and slice
+// ncols, zlo, zhi: as vec2tp_project_mfma; the general kernel (the kit's
+// shape outside mfma_ok, or general set) computes every column and slice
 void vec2tp_project(mlx_ctx *c, const double2 *ur, const double2 *up, const double2 *uz, double2 *psi,
-                    double2 *chi, int nroff, int ncols, int zlo, int zhi, int prec_m0) {
+                    double2 *chi, int nroff, int ncols, int zlo, int zhi, int prec_m0, bool general) {
   const KitDev &k = c->kit;
-  if (c->prec != MLX_PREC_FP64 && mfma_ok(k, 0)) {
+  if (mfma_ok(k, 0) && !general) {
     vec2tp_project_mfma(c, ur, up, uz, psi, chi, ncols, zlo, zhi, prec_m0);
     return;
   }

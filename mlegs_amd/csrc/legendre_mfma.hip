@@ -1,36 +1,30 @@
-// Legendre contractions on MFMA, in FP32 (v_mfma_f32_16x16x4_f32) or FP64
-// (v_mfma_f64_16x16x4_f64).
+// Legendre contractions on MFMA, in FP32 (v_mfma_f32_16x16x4_f32) or
+// split-BF16; the FP64 ones are in legendre_f64.hip.
 //
 // Same contractions as legendre.hip (rtrans_forward / rtrans_backward /
 // vector_projection, src/submodules/mlegs_scalar_ops.f90:1852-2008,
-// 1387-1436).  Fields stay FP64 in HBM; the FP32 kernels round them to FP32
-// when staging into LDS and accumulate in FP32, the FP64 kernels stage and
-// accumulate in FP64 (the same kernels, templated on the operand type).
+// 1387-1436).  Fields stay FP64 in HBM; the kernels round them to FP32 when
+// staging into LDS and accumulate in FP32.
 // These kernels also write every entry of their output (zeros outside the
 // active set), so no separate zero-fill pass is needed.
 //
 // GEMM orientation.  Both directions are computed transposed: the MFMA "A"
 // operand is the field (rows = real columns j = 2k + re/im, contraction
 // dimension in LDS), the "B" operand is the table (columns = radial index).
-// The FP32 instruction's 16x16 accumulator holds rows 4(l/16)+r, column l%16
-// in element r of lane l; the FP64 instruction's holds rows l/16 + 4r
-// (measured on gfx950).  The FP64 kernels feed A row i the field column
-// 4(i%4) + i/4, so in both types element r of lane l holds field column
-// 4(l/16)+r: each lane has the (re, im) pairs of two axial slices for one
-// radial index, and rows 2a and 2a+1 (both parities) or x and nr-1-x are
-// written as contiguous FP64 pairs.
+// The 16x16 accumulator holds rows 4(l/16)+r, column l%16 in element r of lane
+// l: each lane has the (re, im) pairs of two axial slices for one radial
+// index, and rows 2a and 2a+1 (both parities) or x and nr-1-x are written as
+// contiguous FP64 pairs.
 //
 // Work decomposition: one workgroup (4 wavefronts) per (m, 32 axial slices);
 // wave w owns 16-row tiles w, w+4, ... of the radial index.  Contraction in
-// chunks of KC = 8 staged in LDS.
+// chunks of 8 (FP32) or 16 (split-BF16) points staged in LDS.
 #include "mlx_internal.h"
 
 namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef double doublex4 __attribute__((ext_vector_type(4)));
 
-constexpr int KC = 8;         // contraction chunk
 constexpr int KT = 32;        // axial slices per workgroup
 constexpr int BJ = 2 * KT;    // real columns per workgroup
 // LDS row pitches are 16 (mod 64) elements: the four rows an MFMA operand
@@ -70,24 +64,6 @@ struct Mma<float> {
   __device__ static inline vec vzero() { return make_float4(0.f, 0.f, 0.f, 0.f); }
   // field column that A row i carries (accumulator element r of lane l is row 4(l/16)+r)
   __device__ static inline int arow(int i) { return i; }
-};
-template <>
-struct Mma<double> {
-  typedef doublex4 acc;
-  typedef double2 vec;
-  typedef double stage;
-  typedef double pk;
-  static constexpr int VE = 2, KCH = 8, KSTEP = 4, NV = 1;
-  __device__ static inline acc op(double a, double b, acc c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  __device__ static inline pk prep(const stage *v) { return v[0]; }
-  __device__ static inline acc mma(pk a, pk b, acc c) { return op(a, b, c); }
-  __device__ static inline acc zero() { return acc{0.0, 0.0, 0.0, 0.0}; }
-  __device__ static inline vec vzero() { return make_double2(0.0, 0.0); }
-  // accumulator element r of lane l is row l/16 + 4r: A row i carries field
-  // column 4(i%4) + i/4, which puts column 4(l/16)+r in that element
-  __device__ static inline int arow(int i) { return 4 * (i & 3) + (i >> 2); }
 };
 template <>
 struct Mma<Bf3> {
@@ -491,8 +467,7 @@ __global__ void __launch_bounds__(256) k_v2t_mf(const double2 *__restrict__ ur, 
                                                 const T *__restrict__ tgD, const T *__restrict__ tgT,
                                                  const double *__restrict__ ak, int nrdim, int npdim, int nz, int nr,
                                                  int nrh, int nrc0, int npc, int nzc, int nzcu, int nyt, int zlo,
-                                                 int zhi, int mbeg, int mend, int asplit, int tpitch, int ksplit,
-                                                 size_t zso, size_t kstride) {
+                                                 int zhi, int mbeg, int mend, int tpitch) {
   // AP: the table columns (radial rows a of one parity) this workgroup
   // stages; tpitch: the tables' row pitch (4 16 tiles of the widest kernel)
   constexpr int AP = 4 * AT * 16;
@@ -506,21 +481,12 @@ __global__ void __launch_bounds__(256) k_v2t_mf(const double2 *__restrict__ ur, 
   // both parities and every kappa tile of a column m on one XCD: the two
   // parity workgroups read the same input columns and write interleaved
   // rows of the same output lines, which then meet in that XCD's L2
-  // this launch's columns: mbeg .. mend-1.  asplit workgroups share the
-  // rows of one (m, parity, kappa tile): workgroup sp takes the 16-row tiles
-  // wv + 4 (sp AT + s), s < AT, i.e. table columns acol0 .. acol0 + AP - 1
-  // ksplit > 1: workgroup ks contracts the radial points of its share
-  // xb .. xe - 1 only and writes its partial sums to psi/chi + ks kstride
-  // (slice stride zso); a second kernel adds the shares
+  // this launch's columns: mbeg .. mend-1
   int m, y2;
-  xcd_map(blockIdx.x, 2 * nyt * asplit * ksplit, m, y2);
+  xcd_map(blockIdx.x, 2 * nyt, m, y2);
   m += mbeg;
-  const int p = y2 & 1, yt = (y2 >> 1) % nyt, sp = ((y2 >> 1) / nyt) % asplit, ks = ((y2 >> 1) / nyt) / asplit;
+  const int p = y2 & 1, yt = y2 >> 1;
   if (m >= mend) return;
-  const int xshare = ((((nrh + KV - 1) / KV) + ksplit - 1) / ksplit) * KV;
-  const int xb = ks * xshare, xe = (xb + xshare < nrh) ? xb + xshare : nrh;
-  psi += (size_t)ks * kstride;
-  chi += (size_t)ks * kstride;
   const int k0 = yt * KT;
   const int tid = threadIdx.x, lane = tid % 64, wv = tid / 64;
   const size_t zs = (size_t)nrdim * npdim;
@@ -535,8 +501,7 @@ __global__ void __launch_bounds__(256) k_v2t_mf(const double2 *__restrict__ ur, 
   const double2 *cr = ur + (size_t)nrdim * m;
   const double2 *cp = up + (size_t)nrdim * m;
   const double2 *cz = uz + (size_t)nrdim * m;
-  const int acol0 = AP * sp;
-  const size_t tb = ((size_t)m * 2 + p) * nrh * tpitch + acol0;
+  const size_t tb = ((size_t)m * 2 + p) * nrh * tpitch;
   const double seo = (p == 0) ? 1.0 : -1.0;
   typename MM::acc aps[AT][4], ach[AT][4];
 #pragma unroll
@@ -555,8 +520,8 @@ __global__ void __launch_bounds__(256) k_v2t_mf(const double2 *__restrict__ ur, 
   double rkv = 0.0;
   const int fx = tid % KV, fkl = tid / KV;
   if (active) {
-    for (int x0 = xb - KV; x0 < xe; x0 += KV) {
-      if (x0 >= xb) {
+    for (int x0 = -KV; x0 < nrh; x0 += KV) {
+      if (x0 >= 0) {
   #pragma unroll
         for (int j = 0; j < NTV; ++j) {
           const int idx = tid + 256 * j;
@@ -584,7 +549,7 @@ __global__ void __launch_bounds__(256) k_v2t_mf(const double2 *__restrict__ ur, 
         __syncthreads();
       }
       const int xn = x0 + KV;  // chunk fetched now, stored next iteration
-      if (xn < xe) {
+      if (xn < nrh) {
   #pragma unroll
         for (int j = 0; j < NTV; ++j) {
           const int idx = tid + 256 * j;
@@ -593,7 +558,7 @@ __global__ void __launch_bounds__(256) k_v2t_mf(const double2 *__restrict__ ur, 
             const int a = VE * (idx % (AP / VE)), x = (idx / (AP / VE)) % KV, q = idx / ((AP / VE) * KV);
             const int xg = xn + x;
             const T *src = (q == 0) ? tgV : (q == 1) ? tgD : tgT;
-            if (xg < xe) v = *reinterpret_cast<const vec *>(src + tb + (size_t)xg * tpitch + a);
+            if (xg < nrh) v = *reinterpret_cast<const vec *>(src + tb + (size_t)xg * tpitch + a);
           }
           rt[j] = v;
         }
@@ -601,7 +566,7 @@ __global__ void __launch_bounds__(256) k_v2t_mf(const double2 *__restrict__ ur, 
         const double2 z2 = make_double2(0.0, 0.0);
         rra = rrb = rpa = rpb = rza = rzb = z2;
         rkv = 0.0;
-        if (xg < xe && kg < nz) {
+        if (xg < nrh && kg < nz) {
           const size_t oa = (size_t)kg * zs + xg, ob = (size_t)kg * zs + (nr - 1 - xg);
           rra = cr[oa];
           rrb = cr[ob];
@@ -612,7 +577,7 @@ __global__ void __launch_bounds__(256) k_v2t_mf(const double2 *__restrict__ ur, 
           rkv = ak[kg];
         }
       }
-      if (x0 < xb) continue;
+      if (x0 < 0) continue;
   #pragma unroll
       for (int kk = 0; kk < KV; kk += 4) {
         const int xr = kk + lane / 16;
@@ -623,7 +588,7 @@ __global__ void __launch_bounds__(256) k_v2t_mf(const double2 *__restrict__ ur, 
           for (int t = 0; t < 4; ++t) f[q][t] = X[q][xr][16 * t + MM::arow(lane % 16)];
   #pragma unroll
         for (int s = 0; s < AT; ++s) {
-          const int at = wv + 4 * (sp * AT + s);
+          const int at = wv + 4 * s;
           if (at * 16 >= M) continue;
           const int al = (wv + 4 * s) * 16 + lane % 16;  // local table column
           T bv = Tb[0][xr][al];
@@ -644,7 +609,7 @@ __global__ void __launch_bounds__(256) k_v2t_mf(const double2 *__restrict__ ur, 
   }
 #pragma unroll
   for (int s = 0; s < AT; ++s) {
-    const int a = (wv + 4 * (sp * AT + s)) * 16 + lane % 16;
+    const int a = (wv + 4 * s) * 16 + lane % 16;
     const int n = 2 * a + p;
     if (n >= nrdim) continue;
 #pragma unroll
@@ -654,20 +619,19 @@ __global__ void __launch_bounds__(256) k_v2t_mf(const double2 *__restrict__ ur, 
         const int kg = k0 + 8 * t + 2 * (lane / 16) + h;
         if (kg >= nz) continue;
         const bool keep = active && a < M && ((kg + 1 <= nzc) || (kg + 1 >= nzcu)) && !(kg >= zlo && kg <= zhi);
-        size_t o = (size_t)kg * zso + (size_t)nrdim * m + n;
+        size_t o = (size_t)kg * zs + (size_t)nrdim * m + n;
         psi[o] = keep ? make_double2(aps[s][t][2 * h], aps[s][t][2 * h + 1]) : make_double2(0.0, 0.0);
         chi[o] = keep ? make_double2(ach[s][t][2 * h], ach[s][t][2 * h + 1]) : make_double2(0.0, 0.0);
       }
     }
   }
   // rows of this parity past the tiles: zero
-  if (sp != 0) return;  // the first of the row-sharing workgroups zeroes the rest
-  const int A_END = 4 * AT * asplit * 16;
+  const int A_END = 4 * AT * 16;
   const int nrest = (nrdim - p - 2 * A_END + 1) / 2;
   for (int idx = tid; idx < (nrest > 0 ? nrest : 0) * KT; idx += 256) {
     const int n = 2 * (A_END + idx % nrest) + p, kg = k0 + idx / nrest;
     if (kg < nz && n < nrdim) {
-      const size_t o = (size_t)kg * zso + (size_t)nrdim * m + n;
+      const size_t o = (size_t)kg * zs + (size_t)nrdim * m + n;
       psi[o] = make_double2(0.0, 0.0);
       chi[o] = make_double2(0.0, 0.0);
     }
@@ -714,17 +678,20 @@ __global__ void k_tbl_pxa(const double *src, T *dst, int nrh, int rows_per_m, in
 namespace mlx {
 
 int mfma_tiles(const KitDev &k) {
-  // 16-row tiles per wave needed to cover ceil(nrchop/2) rows with 4 waves
+  // groups of 64 rows that cover ceil(nrchop/2) rows of one parity
   int M = (k.nrchop + 1) / 2;
-  int at = (M + 63) / 64;
-  return at;
+  return (M + 63) / 64;
 }
 
+// The largest radial grid of the MFMA kernels: that of the banded solves (544
+// rows).  Above 256 points they run in FP64 whatever the precision (as the
+// general kernels, which such kits took before, do).
+constexpr int kMfmaGroups = 5;
 bool mfma_ok(const KitDev &k, int nroff) {
-  int at = mfma_tiles(k);
-  int xt = (k.nrh + 63) / 64;
-  return nroff == 0 && at >= 1 && at <= 2 && xt >= 1 && xt <= 2;
+  const int at = mfma_tiles(k);
+  return nroff == 0 && at >= 1 && at <= kMfmaGroups && k.nrh <= 64 * kMfmaGroups;
 }
+bool mfma_small(const KitDev &k) { return mfma_tiles(k) <= 2 && k.nrh <= 128; }
 
 void mfma_tables(mlx_ctx *c) {
   KitDev &k = c->kit;
@@ -763,31 +730,34 @@ namespace {
 // the operand type of the MFMA path at the context's current precision:
 // 0 FP32, 1 FP64, 2 split-BF16
 int mfma_kind(const mlx_ctx *c) {
-  if (c->prec == MLX_PREC_FP64_MFMA) return 1;
+  if (!mfma_small(c->kit)) return 1;
+  if (c->prec == MLX_PREC_FP64_MFMA || c->prec == MLX_PREC_FP64) return 1;
   if (c->prec == MLX_PREC_FP32) return 0;
   if (c->prec == MLX_PREC_BF16X3) return 2;
   MLX_THROW(MLX_E_ARG, "MFMA contractions: no kernels for this precision");
 }
-bool mfma_fp64(const mlx_ctx *c) { return mfma_kind(c) == 1; }
 }  // namespace
+bool mfma_fp64(const mlx_ctx *c) { return mfma_kind(c) == 1; }
 
 // ncols > 0: columns m >= ncols are written as zero without being read
 // (ztail = false: they get no workgroups and are left as they are)
-void leg_forward_mfma(mlx_ctx *c, const double2 *in, double2 *out, int ncols, bool ztail) {
+void leg_forward_mfma(mlx_ctx *c, double2 *in, double2 *out, int ncols, bool ztail, const double *ln) {
   const KitDev &k = c->kit;
+  if (mfma_fp64(c)) {
+    const double2 *pin = in;
+    leg_forward_f64(c, &pin, &out, &ln, 1, ncols, ztail);
+    return;
+  }
+  if (ln) k_ln_column(c, in, ln, -1.0);
   const int nyt = (k.nzdim + KT - 1) / KT;
   const int npc = (ncols > 0 && ncols < k.npchop) ? ncols : k.npchop;
   dim3 grid = xcd_grid(ztail ? k.npdim : npc, nyt);
   const int at = mfma_tiles(k);
-  const bool f64 = mfma_fp64(c);
-  ProbeScope probe(c, MLX_PROBE_LEG_FWD, leg_bytes(k, 0, f64 ? 8 : 4, npc), leg_flops(k, 0, npc));
+  ProbeScope probe(c, MLX_PROBE_LEG_FWD, leg_bytes(k, 0, 4, npc), leg_flops(k, 0, npc));
 #define MLX_FWD(T_, AT_, TB_)                                                                                  \
   probed_launch(probe, k_leg_fwd_mf<T_, AT_>, grid, dim3(256), 0, c->stream, in, out, TB_, k.w, k.nrdim, k.npdim, \
                 k.nzdim, k.nr, k.nrh, k.nrchop, npc, nyt)
-  if (f64) {
-    if (at == 1) MLX_FWD(double, 1, k.pfg64);
-    else MLX_FWD(double, 2, k.pfg64);
-  } else if (mfma_kind(c) == 2) {
+  if (mfma_kind(c) == 2) {
     if (at == 1) MLX_FWD(Bf3, 1, k.pfg32);
     else MLX_FWD(Bf3, 2, k.pfg32);
   } else {
@@ -798,22 +768,22 @@ void leg_forward_mfma(mlx_ctx *c, const double2 *in, double2 *out, int ncols, bo
   HIPCHK(hipGetLastError());
 }
 
-void leg_backward_mfma(mlx_ctx *c, const double2 *in, double2 *out, int ncols, bool ztail) {
+void leg_backward_mfma(mlx_ctx *c, const double2 *in, double2 *out, int ncols, bool ztail, const double *ln) {
   const KitDev &k = c->kit;
+  if (mfma_fp64(c)) {
+    leg_backward_f64(c, &in, &out, &ln, 1, ncols, ztail);
+    return;
+  }
   const int nyt = (k.nzdim + KT - 1) / KT;
   const int npc = (ncols > 0 && ncols < k.npchop) ? ncols : k.npchop;
   // without the zero tail only the computed columns get workgroups
   dim3 grid = xcd_grid(ztail ? k.npdim : npc, nyt);
   const int xt = (k.nrh + 63) / 64;
-  const bool f64 = mfma_fp64(c);
-  ProbeScope probe(c, MLX_PROBE_LEG_BWD, leg_bytes(k, 0, f64 ? 8 : 4, npc), leg_flops(k, 0, npc));
+  ProbeScope probe(c, MLX_PROBE_LEG_BWD, leg_bytes(k, 0, 4, npc), leg_flops(k, 0, npc));
 #define MLX_BWD(T_, XT_, TB_)                                                                                    \
   probed_launch(probe, k_leg_bwd_mf<T_, XT_, false>, grid, dim3(256), 0, c->stream, in, out, nullptr, TB_, k.nrdim, \
                 k.npdim, k.nzdim, k.nr, k.nrh, k.ne, k.nrchop, npc, nyt, 0)
-  if (f64) {
-    if (xt == 1) MLX_BWD(double, 1, k.pf);
-    else MLX_BWD(double, 2, k.pf);
-  } else if (mfma_kind(c) == 2) {
+  if (mfma_kind(c) == 2) {
     if (xt == 1) MLX_BWD(Bf3, 1, k.pf32);
     else MLX_BWD(Bf3, 2, k.pf32);
   } else {
@@ -822,6 +792,7 @@ void leg_backward_mfma(mlx_ctx *c, const double2 *in, double2 *out, int ncols, b
   }
 #undef MLX_BWD
   HIPCHK(hipGetLastError());
+  if (ln) k_ln_column(c, out, ln, +1.0);
 }
 
 void leg_backward_pairs_f32(mlx_ctx *c, const double2 *in, float4 *pairs, int ncols) {
@@ -869,7 +840,8 @@ void vec2tp_project_mfma(mlx_ctx *c, const double2 *ur, const double2 *up, const
   if (prec_m0 == MLX_PREC_FP64) prec_m0 = MLX_PREC_FP64_MFMA;  // column 0 stays on MFMA
   // the projection has no split-BF16 kernel: BF16X3 runs it in FP32
   if (prec_m0 == MLX_PREC_BF16X3) prec_m0 = MLX_PREC_FP32;
-  const int prec_rest = c->prec == MLX_PREC_BF16X3 ? MLX_PREC_FP32 : c->prec;
+  const int prec_rest = f64 ? MLX_PREC_FP64_MFMA : MLX_PREC_FP32;
+  if (!mfma_small(k)) prec_m0 = -1;  // FP64 throughout
   const bool split = prec_m0 >= 0 && prec_m0 != prec_rest;
   bool f64_0 = f64;
   if (split) {
@@ -881,53 +853,48 @@ void vec2tp_project_mfma(mlx_ctx *c, const double2 *ur, const double2 *up, const
   const double tb = f64 ? 8.0 : 4.0, tb0 = f64_0 ? 8.0 : 4.0;
   const double bytes = v2t_bytes(k, 0, (int)tb, npc, nzk, true) + 3.0 * k.nrh * nrcs_of(k, 0, 0) * (tb0 - tb);
   ProbeScope probe(c, MLX_PROBE_V2T, bytes, 5.0 * leg_flops(k, 0, npc) * nzk / (double)k.nzdim);
-  // rs: row splits; the launch of column 0 alone spreads its rows over
-  // `at` workgroups of one tile per wave (more workgroups for its long
-  // column, run beside the other columns' launch)
-  // ks > 1: the x contraction in ks shares written to (po, pc), slice
-  // stride nrdim, share stride kst
-  auto launch = [&](bool d, int mb, int me, hipStream_t s, int rs, int ks = 1, double2 *po = nullptr,
-                    double2 *pc = nullptr, size_t kst = 0) {
-    dim3 grid = xcd_grid(me - mb, 2 * nyt * rs * ks);
-    double2 *o0 = ks > 1 ? po : psi, *o1 = ks > 1 ? pc : chi;
-    const size_t zso = ks > 1 ? (size_t)k.nrdim : (size_t)k.nrdim * k.npdim;
-#define MLX_V2T(T_, AT_, V_, D_, T3_)                                                                    \
-  hipLaunchKernelGGL((k_v2t_mf<T_, AT_>), grid, dim3(256), 0, s, ur, up, uz, o0, o1, V_, D_, T3_, k.ak, k.nrdim, \
-                     k.npdim, k.nzdim, k.nr, k.nrh, k.nrchop, npc, k.chopzl, k.chopzu, nyt, zlo, zhi, mb, me, rs, \
-                     k.mfma_ap, ks, zso, kst)
-    const int at_l = rs > 1 ? 1 : at;
+  auto launch = [&](bool d, int mb, int me, hipStream_t s) {
     if (d) {
-      if (at_l == 1) MLX_V2T(double, 1, k.tVg64, k.tDg64, k.tTg64);
-      else MLX_V2T(double, 2, k.tVg64, k.tDg64, k.tTg64);
-    } else {
-      if (at_l == 1) MLX_V2T(float, 1, k.tVg32, k.tDg32, k.tTg32);
-      else MLX_V2T(float, 2, k.tVg32, k.tDg32, k.tTg32);
+      v2t_f64(c, s, ur, up, uz, psi, chi, npc, zlo, zhi, mb, me, 1, (size_t)k.nrdim * k.npdim, 0);
+      return;
     }
+    dim3 grid = xcd_grid(me - mb, 2 * nyt);
+#define MLX_V2T(AT_)                                                                                                \
+  hipLaunchKernelGGL((k_v2t_mf<float, AT_>), grid, dim3(256), 0, s, ur, up, uz, psi, chi, k.tVg32, k.tDg32, k.tTg32, \
+                     k.ak, k.nrdim, k.npdim, k.nzdim, k.nr, k.nrh, k.nrchop, npc, k.chopzl, k.chopzu, nyt, zlo, zhi, \
+                     mb, me, k.mfma_ap)
+    if (at == 1) MLX_V2T(1);
+    else MLX_V2T(2);
 #undef MLX_V2T
     HIPCHK(hipGetLastError());
   };
   probe.mark_start(c->stream);
   if (!split) {
-    launch(f64, 0, k.npdim, c->stream, 1);
+    launch(f64, 0, k.npdim, c->stream);
   } else {
     // fork: column 0 on the second stream once the inputs are ready, the
     // rest on the context stream; join before anything reads psi or chi
     aux_stream_setup(c);
-    // column 0 as 4 shares of its radial points (a quarter of the
+    // column 0 in FP64 as 4 shares of its radial points (a quarter of the
     // contraction's chain each), added in order by a second kernel
     constexpr int KS = 4;
     const size_t kst = (size_t)k.nrdim * k.nzdim;
-    lazy_alloc(c, reinterpret_cast<void **>(&c->v2t_part), sizeof(double2) * 2 * KS * kst,
-               "vector_projection: column-0 shares");
-    double2 *po = c->v2t_part, *pc = c->v2t_part + KS * kst;
+    if (f64_0)
+      lazy_alloc(c, reinterpret_cast<void **>(&c->v2t_part), sizeof(double2) * 2 * KS * kst,
+                 "vector_projection: column-0 shares");
     HIPCHK(hipEventRecord(c->ev_fork, c->stream));
     HIPCHK(hipStreamWaitEvent(c->aux, c->ev_fork, 0));
-    launch(f64_0, 0, 1, c->aux, at, KS, po, pc, kst);
-    hipLaunchKernelGGL(k_v2t_col0_sum, dim3((unsigned)((kst + 255) / 256 < 1024 ? (kst + 255) / 256 : 1024)),
-                       dim3(256), 0, c->aux, psi, chi, po, pc, KS, kst, k.nrdim, k.nzdim,
-                       (size_t)k.nrdim * k.npdim);
-    HIPCHK(hipGetLastError());
-    launch(f64, 1, k.npdim, c->stream, 1);
+    if (f64_0) {
+      double2 *po = c->v2t_part, *pc = c->v2t_part + KS * kst;
+      v2t_f64(c, c->aux, ur, up, uz, po, pc, npc, zlo, zhi, 0, 1, KS, (size_t)k.nrdim, kst);
+      hipLaunchKernelGGL(k_v2t_col0_sum, dim3((unsigned)((kst + 255) / 256 < 1024 ? (kst + 255) / 256 : 1024)),
+                         dim3(256), 0, c->aux, psi, chi, po, pc, KS, kst, k.nrdim, k.nzdim,
+                         (size_t)k.nrdim * k.npdim);
+      HIPCHK(hipGetLastError());
+    } else {
+      launch(false, 0, 1, c->aux);
+    }
+    launch(f64, 1, k.npdim, c->stream);
     HIPCHK(hipEventRecord(c->ev_join, c->aux));
     HIPCHK(hipStreamWaitEvent(c->stream, c->ev_join, 0));
   }

@@ -340,16 +340,30 @@ void fft_z_batch(mlx_ctx *c, double2 *const *e, int nf, int dir, double ncol, in
 // ncols > 0 (MFMA path): only columns m < ncols are transformed, the others
 // are written as zero (their input is zero or their output unused)
 // ztail = false (MFMA path): columns m >= ncols are left unwritten
-void leg_forward(mlx_ctx *c, const double2 *in, double2 *out, int nroff, bool zero = true, int ncols = -1,
-                 bool ztail = true);
+// ln (optional): the field's log coefficient (device): the forward transform
+// takes the input less ln ln x in column 0 (other than the FP64 MFMA kernels
+// change the input itself), the backward one adds it to the output
+void leg_forward(mlx_ctx *c, double2 *in, double2 *out, int nroff, bool zero = true, int ncols = -1,
+                 bool ztail = true, const double *ln = nullptr);
 void leg_backward(mlx_ctx *c, const double2 *in, double2 *out, int nroff, bool zero = true, int ncols = -1,
-                  bool ztail = true);
-// legendre_mfma.hip (MFMA in FP32 or FP64 by c->prec; valid when mfma_ok)
+                  bool ztail = true, const double *ln = nullptr);
+// legendre_mfma.hip (MFMA at c->prec; valid when mfma_ok)
 bool mfma_ok(const KitDev &k, int nroff);
+bool mfma_small(const KitDev &k);  // the FP32 and split-BF16 kernels cover the kit
+bool mfma_fp64(const mlx_ctx *c);  // the MFMA contractions run in FP64
 void mfma_tables(mlx_ctx *c);
-void leg_forward_mfma(mlx_ctx *c, const double2 *in, double2 *out, int ncols = -1, bool ztail = true);
-// ztail = false: columns m >= ncols are left unwritten
-void leg_backward_mfma(mlx_ctx *c, const double2 *in, double2 *out, int ncols = -1, bool ztail = true);
+void leg_forward_mfma(mlx_ctx *c, double2 *in, double2 *out, int ncols = -1, bool ztail = true,
+                      const double *ln = nullptr);
+void leg_backward_mfma(mlx_ctx *c, const double2 *in, double2 *out, int ncols = -1, bool ztail = true,
+                       const double *ln = nullptr);
+// legendre_f64.hip: the FP64 ones of the nf (<= kZBatch) fields in[] -> out[]
+// in one launch, ln null or one pointer (or null) per field
+void leg_forward_f64(mlx_ctx *c, const double2 *const *in, double2 *const *out, const double *const *ln, int nf,
+                     int ncols = -1, bool ztail = true);
+void leg_backward_f64(mlx_ctx *c, const double2 *const *in, double2 *const *out, const double *const *ln, int nf,
+                      int ncols = -1, bool ztail = true);
+void v2t_f64(mlx_ctx *c, hipStream_t s, const double2 *ur, const double2 *up, const double2 *uz, double2 *psi,
+             double2 *chi, int npc, int zlo, int zhi, int mbeg, int mend, int ksplit, size_t zso, size_t kstride);
 // the FP32 even/odd sums (be, bo) of columns m < ncols as float4 radial pairs
 // (layout at k_leg_bwd_f32), for fft_phi_pairs; a line of pairs (one z slice
 // and column) takes pair_stride float4 (256-byte aligned lines)
@@ -360,7 +374,7 @@ void vec2tp_project_mfma(mlx_ctx *c, const double2 *ur, const double2 *up, const
                          double2 *chi, int ncols = -1, int zlo = 1, int zhi = 0, int prec_m0 = -1);
 void vec2tp_project(mlx_ctx *c, const double2 *ur, const double2 *up, const double2 *uz,
                     double2 *psi, double2 *chi, int nroff, int ncols = -1,
-                    int zlo = 1, int zhi = 0, int prec_m0 = -1);
+                    int zlo = 1, int zhi = 0, int prec_m0 = -1, bool general = false);
 
 // spectral.hip
 void k_ln_column(mlx_ctx *c, double2 *e, const double *ln, double sign);
