@@ -452,63 +452,76 @@ void abcn_pair(mlx_ctx *c, mlx_field *s1, mlx_field *s1p, mlx_field *nl1, mlx_fi
   fmove(nl2p, nl2);
 }
 
-// tp2vec_back's z transforms of the nf fields f[0..nf) in one launch
-void tp2vec_back_z(mlx_ctx *c, mlx_field *const *f, int nf, int ncols, int zlo, int zhi) {
+// The backward (forward) radial transform of the nf fields f[0..nf), offset 0:
+// one launch in place on the FP64 MFMA path, else one launch each.  nc, ztail:
+// leg_backward's ncols and ztail.
+void leg_n(mlx_ctx *c, mlx_field *const *f, int nf, bool backward, int nc, bool ztail) {
   const KitDev &k = c->kit;
-  if (k.nz <= 1) return;
-  const int nc = (ncols > 0 && ncols < k.npchop) ? ncols : k.npchop;
-  double2 *e[kZBatch];
-  for (int q = 0; q < nf; ++q) e[q] = f[q]->e;
-  fft_z_batch(c, e, nf, +1, active_pairs(k, 0, nc), k.nrchop, nc, zlo, zhi);
+  if (mfma_ok(k, 0) && mfma_fp64(c) && leg_inplace_ok(k)) {
+    double2 *e[kZBatch];
+    for (int q = 0; q < nf; ++q) e[q] = f[q]->e;
+    (backward ? leg_backward_f64 : leg_forward_f64)(c, e, e, nullptr, nf, nc, ztail);
+    return;
+  }
+  for (int q = 0; q < nf; ++q) {
+    if (backward) leg_backward(c, f[q]->e, c->scr[0], 0, true, nc, ztail);
+    else leg_forward(c, f[q]->e, c->scr[0], 0, true, nc, ztail);
+    swap_scr(c, f[q]);
+  }
 }
 
-// Back half of tp2vec: the three FFF components (offset 0, no log term) to
-// PPP; ur and up are divided by r in the last phi transform.  ncols > 0: the
-// components are zero in columns m >= ncols, which the transforms skip.
+// Back half of tp2vec for nf = 3 or 6 fields, (u_r, u_phi, u_z) each: the FFF
+// components (offset 0, no log term) to PPP; u_r and u_phi are divided by r in
+// the last phi transform.  ncols > 0: the components are zero in columns m >=
+// ncols, which the transforms skip; slices zlo..zhi of the input are zero.
 // The front kernel has zeroed the log terms, so trans's log-column step
-// (adding 0 * ln x) is left out; the other steps are trans's FFF -> PPP.
+// (adding 0 * ln x) is left out; the other steps are trans's FFF -> PPP.  Each
+// of the three transforms is one launch for all the fields, except the radial
+// pairs' (270 MB of pairs at 256^3 would not stay in the last-level cache).
 // phys_rows: rows nr.. of the outputs are not needed (the caller's cross
 // product takes them as zero) and are not synthesized
 // f32_ok: the caller reads the outputs through fft_phi_cross's FP32 input;
 // when the radial pairs path runs (FP32 sums) the outputs are then stored in
-// FP32.  Returns whether they were.
-// z_done: the caller has run the z transforms (tp2vec_back_z)
-bool tp2vec_back(mlx_ctx *c, mlx_field *ur, mlx_field *up, mlx_field *uz, int ncols = -1, int zlo = 1,
-                 int zhi = 0, bool phys_rows = false, bool f32_ok = false, bool z_done = false) {
+// FP32.  Returns how they were stored: 2 in FP32, 1 in FP64, 0 in FP64 from
+// FP32 sums.
+int tp2vec_back(mlx_ctx *c, mlx_field *const *f, int nf, int ncols = -1, int zlo = 1, int zhi = 0,
+                bool phys_rows = false, bool f32_ok = false) {
   const KitDev &k = c->kit;
   PrecScope ps(c, MLX_STAGE_SYNTH);
-  const int rs[3] = {-1, -1, 0};
+  const int rs[6] = {-1, -1, 0, -1, -1, 0};
   const int nc = (ncols > 0 && ncols < k.npchop) ? ncols : k.npchop;
-  // limited columns and the four-step phi kernels: the radial transform
-  // leaves columns m >= nc unwritten and the phi transform takes them as zero
-  const bool lean = nc < k.npchop && fft_phi_fast(k);
+  // limited columns: the radial transform leaves columns m >= nc unwritten and
+  // the phi transform takes them as zero
+  const bool lean = nc < k.npchop && k.np > 1;
   // physical rows only, on the MFMA path: the radial transform hands the
   // phi transform its FP32 even/odd sums (half the bytes of the FP64 rows,
   // which the phi transform forms from them exactly)
-  const bool pairs = lean && phys_rows && (c->prec == MLX_PREC_FP32 || c->prec == MLX_PREC_BF16X3) && mfma_ok(k, 0) &&
-                     mfma_small(k);
-  // the de-aliased kappa slices zlo..zhi of the input are zero
-  mlx_field *const three[3] = {ur, up, uz};
-  if (!z_done) tp2vec_back_z(c, three, 3, ncols, zlo, zhi);
-  int q = 0;
-  for (mlx_field *f : three) {
-    f->off[0] = f->off[1] = f->off[2] = 0;
-    if (pairs) {
-      float4 *pr = reinterpret_cast<float4 *>(c->scr[0]);
-      leg_backward_pairs_f32(c, f->e, pr, nc);
-      fft_phi_pairs(c, f->e, pr, rs[q], nc, f32_ok);
-      set_space(f, "PPP");
-      ++q;
-      continue;
-    }
-    leg_backward(c, f->e, c->scr[0], 0, true, nc, !lean);
-    swap_scr(c, f);
-    if (k.np > 1) fft_phi(c, f->e, f->e, +1, rs[q], lean ? nc : -1, phys_rows && fft_phi_fast(k));
-    else if (rs[q] < 0) k_scale_rows_r(c, f->e, 1);
-    set_space(f, "PPP");
-    ++q;
+  const bool fp32 = mfma_ok(k, 0) && !mfma_fp64(c);
+  const bool pairs = lean && phys_rows && fp32;
+  double2 *e[kZBatch];
+  for (int q = 0; q < nf; ++q) {
+    e[q] = f[q]->e;
+    f[q]->off[0] = f[q]->off[1] = f[q]->off[2] = 0;
   }
-  return pairs && f32_ok;
+  if (k.nz > 1) fft_z_batch(c, e, nf, +1, active_pairs(k, 0, nc), k.nrchop, nc, zlo, zhi);
+  if (pairs) {
+    const bool f32 = f32_ok && fft_f32_rows(k);
+    float4 *pr = reinterpret_cast<float4 *>(c->scr[0]);
+    for (int q = 0; q < nf; ++q) {
+      leg_backward_pairs_f32(c, f[q]->e, pr, nc);
+      fft_phi_pairs(c, f[q]->e, pr, rs[q], nc, f32);
+      set_space(f[q], "PPP");
+    }
+    return f32 ? 2 : 0;
+  }
+  leg_n(c, f, nf, true, nc, !lean);
+  for (int q = 0; q < nf; ++q) {
+    e[q] = f[q]->e;
+    set_space(f[q], "PPP");
+    if (k.np <= 1 && rs[q] < 0) k_scale_rows_r(c, f[q]->e, 1);
+  }
+  fft_phi_batch(c, e, e, nf, +1, rs, lean ? nc : -1, phys_rows);
+  return fp32 ? 0 : 1;
 }
 
 // tp2vec (vector_reconstruction, mlegs_scalar_ops.f90:1455-1545): the +3-offset
@@ -519,11 +532,11 @@ void tp2vec(mlx_ctx *c, const mlx_field *psi, const mlx_field *chi, mlx_field *v
   need_kit(c);
   if (!is_fff(psi) || !is_fff(chi)) MLX_THROW(MLX_E_LAYOUT, "vector_projection: psi and chi must be in FFF");
   mlx_field *ur = tmp(c, 0), *up = tmp(c, 1), *uz = tmp(c, 2);
-  // the z transform of tp2vec_back takes zlo..zhi as zero (four-step kernels)
-  const bool zskip = fft_z_fast(c->kit);
-  k_tp2vec_front(c, ur->e, up->e, uz->e, psi->e, chi->e, psi->sc, chi->sc, 0, 0, ur->sc, up->sc, uz->sc, ncols,
-                 zskip ? zlo : 1, zskip ? zhi : 0);
-  tp2vec_back(c, ur, up, uz, ncols, zlo, zhi);
+  // the z transform of tp2vec_back takes zlo..zhi as zero
+  k_tp2vec_front(c, ur->e, up->e, uz->e, psi->e, chi->e, psi->sc, chi->sc, 0, 0, ur->sc, up->sc, uz->sc, ncols, zlo,
+                 zhi);
+  mlx_field *const three[3] = {ur, up, uz};
+  tp2vec_back(c, three, 3, ncols, zlo, zhi);
   fmove(vr, ur);
   fmove(vp, up);
   fmove(vz, uz);
@@ -537,10 +550,10 @@ void tp2curlvec(mlx_ctx *c, const mlx_field *psi, const mlx_field *chi, mlx_fiel
   if (!is_fff(psi) || !is_fff(chi)) MLX_THROW(MLX_E_LAYOUT, "vector_projection: psi and chi must be in FFF");
   mlx_field *ur = tmp(c, 0), *up = tmp(c, 1), *uz = tmp(c, 2);
   // del2 of md = chi runs over the rows of chi's own radial offset
-  const bool zskip = fft_z_fast(c->kit);
   k_tp2vec_front(c, ur->e, up->e, uz->e, chi->e, psi->e, chi->sc, psi->sc, 1, chi->off[0], ur->sc, up->sc,
-                 uz->sc, ncols, zskip ? zlo : 1, zskip ? zhi : 0);
-  tp2vec_back(c, ur, up, uz, ncols, zlo, zhi);
+                 uz->sc, ncols, zlo, zhi);
+  mlx_field *const three[3] = {ur, up, uz};
+  tp2vec_back(c, three, 3, ncols, zlo, zhi);
   fmove(wr, ur);
   fmove(wp, up);
   fmove(wz, uz);
@@ -572,7 +585,7 @@ void adj_no_offsets(const mlx_field *f, const char *what) {
 // side; the diagonal factors run as one pass.  to_fff: g in PPP holds the
 // cotangent of r^rmode B(x) and returns that of x, in FFF; otherwise g in
 // FFF holds the cotangent of F(r^rmode y) and returns that of y, in PPP.
-// lim (optional, with the four-step phi kernels): the FFF side is de-aliased
+// lim (optional): the FFF side is de-aliased
 // (columns m >= pcut and slices zlo..zhi zero on input, or not needed on
 // output: to_fff leaves them unwritten).  The nf (<= kZBatch) fields gs[q]
 // (row factors rmodes[q]) share one launch of the z transform.
@@ -595,26 +608,23 @@ void trans_adjoint_nolog_n(mlx_ctx *c, mlx_field *const *gs, int nf, bool to_fff
   };
   if (to_fff) {
     // B^T = Z_b^T L_b^T Phi_b^T (L_b^T = L_f W^-1, Z_b^T = nz Z_f)
-    for (int q = 0; q < nf; ++q) {
-      mlx_field *g = gs[q];
-      if (k.np > 1) fft_phi(c, g->e, g->e, -1);
-      k_adj_diag(c, g->e, -1, rmodes[q], k.np > 1 ? +1 : 0, k.nz > 1 ? (double)k.nz : 1.0);
-      leg_forward(c, g->e, c->scr[0], 0, true, nc, !lim);
-      swap_scr(c, g);
-    }
+    for (int q = 0; q < nf; ++q) e[q] = gs[q]->e;
+    fft_phi_batch(c, e, e, nf, -1);
+    for (int q = 0; q < nf; ++q)
+      k_adj_diag(c, gs[q]->e, -1, rmodes[q], k.np > 1 ? +1 : 0, k.nz > 1 ? (double)k.nz : 1.0);
+    leg_n(c, gs, nf, false, nc, !lim);
     z(-1);
     for (int q = 0; q < nf; ++q) set_space(gs[q], "FFF");
   } else {
     // F^T = Phi_f^T L_f^T Z_f^T (L_f^T = W L_b, Z_f^T = Z_b / nz)
     z(+1);
+    leg_n(c, gs, nf, true, nc, !lim);
     for (int q = 0; q < nf; ++q) {
-      mlx_field *g = gs[q];
-      leg_backward(c, g->e, c->scr[0], 0, true, nc, !lim);
-      swap_scr(c, g);
-      k_adj_diag(c, g->e, +1, rmodes[q], k.np > 1 ? -1 : 0, k.nz > 1 ? 1.0 / k.nz : 1.0);
-      if (k.np > 1) fft_phi(c, g->e, g->e, +1, 0, lim ? lim->pcut : -1);
-      set_space(g, "PPP");
+      k_adj_diag(c, gs[q]->e, +1, rmodes[q], k.np > 1 ? -1 : 0, k.nz > 1 ? 1.0 / k.nz : 1.0);
+      e[q] = gs[q]->e;
+      set_space(gs[q], "PPP");
     }
+    fft_phi_batch(c, e, e, nf, +1, nullptr, lim ? lim->pcut : -1);
   }
 }
 
@@ -772,12 +782,13 @@ void pff_adjoint_n(mlx_ctx *c, mlx_field *const *gs, int nf, const int *rmodes, 
     else
       fft_z_batch(c, e, nf, +1, (double)k.nrdim * k.npdim);
   }
+  double2 *e[kZBatch];
   for (int q = 0; q < nf; ++q) {
-    mlx_field *g = gs[q];
-    k_adj_diag(c, g->e, 0, rmodes[q], k.np > 1 ? -1 : 0, k.nz > 1 ? 1.0 / k.nz : 1.0);
-    if (k.np > 1) fft_phi(c, g->e, g->e, +1, 0, lim ? lim->pcut : -1);
-    set_space(g, "PPP");
+    k_adj_diag(c, gs[q]->e, 0, rmodes[q], k.np > 1 ? -1 : 0, k.nz > 1 ? 1.0 / k.nz : 1.0);
+    e[q] = gs[q]->e;
+    set_space(gs[q], "PPP");
   }
+  fft_phi_batch(c, e, e, nf, +1, nullptr, lim ? lim->pcut : -1);
 }
 
 // tp2vec's transpose (vector_reconstruction, mlegs_scalar_ops.f90:1455-1545):
@@ -905,15 +916,12 @@ void advection_adjoint(mlx_ctx *c, mlx_field *psi, mlx_field *chi, const mlx_fie
     // v and w at (psi, chi): the fused column pass and the backward
     // transforms of advection_rhs, skipping what de-aliasing zeroes, in FP64
     const int ncols = dl.on ? dl.pcut : -1;
-    const bool zskip = fft_z_fast(c->kit);
     mlx_field *vr = tmp(c, 24), *vp = tmp(c, 25), *vz = tmp(c, 26);
     mlx_field *wr = tmp(c, 27), *wp = tmp(c, 28), *wz = tmp(c, 29);
     k_tp2vec_front2(c, vr->e, vp->e, vz->e, vr->sc, vp->sc, vz->sc, wr->e, wp->e, wz->e, wr->sc, wp->sc, wz->sc,
-                    psi->e, chi->e, psi->sc, chi->sc, chi->off[0], ncols, zskip ? dl.zlo : 1, zskip ? dl.zhi : 0);
+                    psi->e, chi->e, psi->sc, chi->sc, chi->off[0], ncols, dl.zlo, dl.zhi);
     mlx_field *const six[6] = {vr, vp, vz, wr, wp, wz};
-    tp2vec_back_z(c, six, 6, ncols, dl.zlo, dl.zhi);
-    tp2vec_back(c, vr, vp, vz, ncols, dl.zlo, dl.zhi, true, false, true);
-    tp2vec_back(c, wr, wp, wz, ncols, dl.zlo, dl.zhi, true, false, true);
+    tp2vec_back(c, six, 6, ncols, dl.zlo, dl.zhi, true);
     v[0] = vr->e, v[1] = vp->e, v[2] = vz->e;
     w[0] = wr->e, w[1] = wp->e, w[2] = wz->e;
   }
@@ -921,9 +929,8 @@ void advection_adjoint(mlx_ctx *c, mlx_field *psi, mlx_field *chi, const mlx_fie
   set_space(nlchib, "FFF");
   dealias(c, nlpsib);
   dealias(c, nlchib);
-  // the transforms below skip the de-aliased modes (the four-step phi
-  // kernels take the mode limit)
-  const DealiasLimits *lim = (dl.on && fft_phi_fast(c->kit)) ? &dl : nullptr;
+  // the transforms below skip the de-aliased modes
+  const DealiasLimits *lim = dl.on ? &dl : nullptr;
   mlx_field *ar = tmp(c, 30), *ap = tmp(c, 31), *az = tmp(c, 32);
   vec2tp_adjoint(c, nlpsib, nlchib, ar, ap, az, lim);
   // (v + U) x w: v_b = w x a, w_b = a x (v + U)
@@ -1065,38 +1072,31 @@ int advection_rhs(mlx_ctx *c, mlx_field *psi, mlx_field *chi, mlx_field *nlpsi, 
   // psi and chi are de-aliased here and so is the result: the MFMA path
   // skips the columns and slices de-aliasing zeroes
   const DealiasLimits dl = general_projection(c, nlchi) ? DealiasLimits() : dealias_limits(c);
-  bool f32phys = false;
-  {
-    // tp2vec and tp2curlvec: both front passes in one launch, then the six
-    // backward transforms
-    const int ncols = dl.on ? dl.pcut : -1;
-    const bool zskip = fft_z_fast(c->kit);
-    k_tp2vec_front2(c, vr->e, vp->e, vz->e, vr->sc, vp->sc, vz->sc, wr->e, wp->e, wz->e, wr->sc, wp->sc, wz->sc,
-                    psi->e, chi->e, psi->sc, chi->sc, chi->off[0], ncols, zskip ? dl.zlo : 1, zskip ? dl.zhi : 0);
-    // the six physical fields are read only by the fused cross-product
-    // transform below: with FP32 radial sums they are stored in FP32
-    const bool cross = fft_phi_cross_ok(c->kit);
-    // the six z transforms in one launch
-    mlx_field *const six[6] = {vr, vp, vz, wr, wp, wz};
-    tp2vec_back_z(c, six, 6, ncols, dl.zlo, dl.zhi);
-    f32phys = tp2vec_back(c, vr, vp, vz, ncols, dl.zlo, dl.zhi, true, cross, true);
-    if (tp2vec_back(c, wr, wp, wz, ncols, dl.zlo, dl.zhi, true, cross, true) != f32phys)
-      MLX_THROW(MLX_E_ARG, "advection_rhs: velocity and vorticity stored at different precisions");
-  }
+  // tp2vec and tp2curlvec: both front passes in one launch, then the six
+  // backward transforms; the six physical fields are read only by the fused
+  // cross-product transform below (with FP32 radial sums they are stored in
+  // FP32)
+  const int ncols = dl.on ? dl.pcut : -1;
+  k_tp2vec_front2(c, vr->e, vp->e, vz->e, vr->sc, vp->sc, vz->sc, wr->e, wp->e, wz->e, wr->sc, wp->sc, wz->sc,
+                  psi->e, chi->e, psi->sc, chi->sc, chi->off[0], ncols, dl.zlo, dl.zhi);
+  mlx_field *const six[6] = {vr, vp, vz, wr, wp, wz};
+  const bool cross = c->kit.np > 1;
+  const int fmt = tp2vec_back(c, six, 6, ncols, dl.zlo, dl.zhi, cross, cross);
   // de-aliased inside vec2tp before idel2; chop and zeroat1 keep zero modes
   // zero, so the closing dealias of the reference is already satisfied
   mlx_field *ur = tmp(c, 0), *up = tmp(c, 1), *uzp = tmp(c, 2);
-  if (fft_phi_cross(c, ur->e, up->e, uzp->e, vr->e, vp->e, vz->e, wr->e, wp->e, wz->e, uz->e, ur->sc, up->sc,
-                    uzp->sc, dl.on ? dl.pcut : -1, f32phys)) {
+  if (cross) {
     // vz + uz, v x w, and the phi transforms of r (v x w)_r, r (v x w)_phi,
     // (v x w)_z in one pass: log terms zero (set by the kernel), no offsets,
     // as vecprod leaves them
+    fft_phi_cross(c, ur->e, up->e, uzp->e, vr->e, vp->e, vz->e, wr->e, wp->e, wz->e, uz->e, ur->sc, up->sc, uzp->sc,
+                  dl.on ? dl.pcut : -1, fmt == 2);
     for (mlx_field *f : {ur, up, uzp}) {
       f->off[0] = f->off[1] = f->off[2] = 0;
       set_space(f, "PFP");
     }
     vec2tp_pfp(c, ur, up, uzp, nlpsi, nlchi, true, dl, true);
-    return f32phys ? 2 : 1;
+    return fmt;
   }
   k_axpby(c, vz->e, vz->sc, 1.0, uz->e, nullptr, 1.0);
   vecprod(c, vr, vp, vz, wr, wp, wz);
@@ -1930,7 +1930,9 @@ int mlx_time_kernel(mlx_ctx *c, mlx_field *f, const char *which, int32_t iters, 
       else if (w == "v2t") vec2tp_project(c, f->e, f->e, f->e, c->scr[0], c->scr[1], 3);
       else if (w == "lu_solve") k_helm_solve(c, f->e, -2.0 / (c->p.dt * c->p.visc), 0, 0);
       else if (w == "phi_cross") {
-        if (!fft_phi_cross(c, tmp(c, 0)->e, tmp(c, 1)->e, tmp(c, 2)->e, f->e, f->e, f->e, f->e, f->e, f->e, f->e))
+        if (c->kit.np > 1)
+          fft_phi_cross(c, tmp(c, 0)->e, tmp(c, 1)->e, tmp(c, 2)->e, f->e, f->e, f->e, f->e, f->e, f->e, f->e);
+        else
           MLX_THROW(MLX_E_ARG, "mlx_time_kernel: phi_cross is not built for this np");
       }
       else if (w == "copy") k_copy_field(c, c->scr[0], f->e);

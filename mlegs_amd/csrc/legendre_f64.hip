@@ -507,6 +507,10 @@ LegFields leg_fields(const double2 *const *in, double2 *const *out, const double
 
 namespace mlx {
 
+// In place: one workgroup then reads all of a column's slices it writes, and
+// has read them before it writes the first.
+bool leg_inplace_ok(const KitDev &k) { return k.nrh <= 128 && (k.nrchop + 1) / 2 <= 128; }
+
 // ncols > 0: columns m >= ncols are written as zero without being read
 // (ztail = false: they get no workgroups and are left as they are)
 void leg_forward_f64(mlx_ctx *c, const double2 *const *in, double2 *const *out, const double *const *ln, int nf,
@@ -520,7 +524,9 @@ void leg_forward_f64(mlx_ctx *c, const double2 *const *in, double2 *const *out, 
   // to a CU; 16 slices and 64 rows below (256^3: 101 us against 118; 128 x 64
   // x 64, 66 workgroups of the large kind: 12.4 against 7.4 us)
   const LegDims big = leg_dims(k, nf, npc, ncol, 32, (M + 127) / 128);
-  if (npc * big.nyt * big.nsp >= 512) {
+  const bool inplace = in[0] == out[0];
+  if (inplace && !leg_inplace_ok(k)) MLX_THROW(MLX_E_ARG, "rtrans_forward: in place past 256 radial points");
+  if (npc * big.nyt * big.nsp >= 512 || (inplace && M > 64)) {
     probed_launch(probe, k_leg_fwd_f64m<32, 2, 8>, dim3(ncol * big.nyt * big.nsp), dim3(512), 0, c->stream, f, big,
                   (const double *)k.pfg64);
   } else {
@@ -538,6 +544,7 @@ void leg_backward_f64(mlx_ctx *c, const double2 *const *in, double2 *const *out,
   const LegFields f = leg_fields(in, out, ln, nf);
   ProbeScope probe(c, MLX_PROBE_LEG_BWD, nf * leg_bytes(k, 0, 8, npc), nf * leg_flops(k, 0, npc));
   const LegDims d = leg_dims(k, nf, npc, ncol, 16, (k.nrh + 127) / 128);
+  if (in[0] == out[0] && d.nsp > 1) MLX_THROW(MLX_E_ARG, "rtrans_backward: in place past 256 radial points");
   probed_launch(probe, k_leg_bwd_f64m, dim3(ncol * d.nyt * d.nsp), dim3(512), 0, c->stream, f, d, (const double *)k.pf);
   HIPCHK(hipGetLastError());
 }

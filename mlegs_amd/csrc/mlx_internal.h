@@ -295,44 +295,42 @@ void kit_build(mlx_ctx *c);
 void kit_free(KitDev &k);
 
 // fft.hip
+constexpr int kZBatch = 6;  // fields per batched launch (transforms, contractions)
 // dir -1 forward (PPP->PFP), +1 backward; out may equal in; rscale: +1 multiply
 // input rows i < nr by r_i (forward), -1 divide output rows by r_i (backward)
-// mlim > 0 (backward, fast path only): modes m >= mlim are taken as zero
-// without being read
-// phys_rows (backward, fast path): only rows i < nr are synthesized and
-// written (rows nr.. of the output are left as they are)
+// mlim > 0 (backward): modes m >= mlim are taken as zero without being read
+// phys_rows (backward): only rows i < nr are synthesized and written (rows
+// nr.. of the output are left as they are)
 void fft_phi(mlx_ctx *c, double2 *out, const double2 *in, int dir, int rscale = 0, int mlim = -1,
              bool phys_rows = false);
+// the same of the nf (<= kZBatch) fields in[] -> out[] in one launch (rscale:
+// one per field, or null)
+void fft_phi_batch(mlx_ctx *c, double2 *const *out, const double2 *const *in, int nf, int dir,
+                   const int *rscale = nullptr, int mlim = -1, bool phys_rows = false);
 // backward phi transform of leg_backward_pairs_f32's radial pairs into rows
-// < nr of out (fast path only)
+// < nr of out
 // f32out: the rows are stored in FP32 (float pair e of out's buffer for
-// entry e), for fft_phi_cross's FP32 input
+// entry e), for fft_phi_cross's FP32 input (where fft_f32_rows holds)
 void fft_phi_pairs(mlx_ctx *c, double2 *out, const float4 *pairs, int rscale, int mlim, bool f32out = false);
-bool fft_phi_fast(const KitDev &k);  // the four-step phi kernels cover np/2
-bool fft_z_fast(const KitDev &k);    // the four-step z kernels cover nz
+bool fft_f32_rows(const KitDev &k);  // the kernels with FP32 physical fields cover np/2
 // v x w (v_z + ub) to PFP with the r weights of vector_projection (modes
-// m < mmax written; mmax <= 0: all); false when
-// the fused form is not built for this np (the caller then runs vecprod and
-// three phi transforms)
+// m < mmax written; mmax <= 0: all), np > 1
 // f32in: v0..w2 are stored in FP32 (as fft_phi_pairs's f32out writes them)
-bool fft_phi_cross(mlx_ctx *c, double2 *o0, double2 *o1, double2 *o2, const double2 *v0, const double2 *v1,
+void fft_phi_cross(mlx_ctx *c, double2 *o0, double2 *o1, double2 *o2, const double2 *v0, const double2 *v1,
                    const double2 *v2, const double2 *w0, const double2 *w1, const double2 *w2, const double2 *ub,
                    double *ln0 = nullptr, double *ln1 = nullptr, double *ln2 = nullptr, int mmax = -1,
                    bool f32in = false);
-bool fft_phi_cross_ok(const KitDev &k);  // the fused kernel is built for this np
 // dir -1 forward (/nz), +1 backward.  ncol: the (row, column) lines the caller
 // needs transformed (the launch's algorithmic work).  act_nrc > 0: only rows
 // i < act_nrc - j of column j need transforming; ncols > 0: only columns
 // j < ncols.  Lines outside are left as they are (the caller guarantees they
-// are zero or never read); the generic kernel transforms every line.
+// are zero or never read).
 // zin_lo..zin_hi: line entries known to be zero (not read); zout_lo..zout_hi:
-// outputs the caller does not use (not written) -- four-step kernels only,
-// the generic kernel reads and writes everything
+// outputs the caller does not use (not written)
 void fft_z(mlx_ctx *c, double2 *e, int dir, double ncol, int act_nrc = 0, int ncols = 0, int zin_lo = 1,
            int zin_hi = 0, int zout_lo = 1, int zout_hi = 0);
 // the same transform of the nf (<= kZBatch) fields e[0..nf) in one launch
 // (ncol: per field)
-constexpr int kZBatch = 6;
 void fft_z_batch(mlx_ctx *c, double2 *const *e, int nf, int dir, double ncol, int act_nrc = 0, int ncols = 0,
                  int zin_lo = 1, int zin_hi = 0, int zout_lo = 1, int zout_hi = 0);
 
@@ -357,7 +355,9 @@ void leg_forward_mfma(mlx_ctx *c, double2 *in, double2 *out, int ncols = -1, boo
 void leg_backward_mfma(mlx_ctx *c, const double2 *in, double2 *out, int ncols = -1, bool ztail = true,
                        const double *ln = nullptr);
 // legendre_f64.hip: the FP64 ones of the nf (<= kZBatch) fields in[] -> out[]
-// in one launch, ln null or one pointer (or null) per field
+// in one launch, ln null or one pointer (or null) per field.  out[] may be
+// in[] where leg_inplace_ok holds.
+bool leg_inplace_ok(const KitDev &k);
 void leg_forward_f64(mlx_ctx *c, const double2 *const *in, double2 *const *out, const double *const *ln, int nf,
                      int ncols = -1, bool ztail = true);
 void leg_backward_f64(mlx_ctx *c, const double2 *const *in, double2 *const *out, const double *const *ln, int nf,
