@@ -425,8 +425,8 @@ __global__ void __launch_bounds__(kThreads) k_fftg(FftgArgs a) {
 // padded to 128-byte lines, half the bytes).
 // gridDim.z > 1: the fields f.in[z] -> f.out[z] (same shape and limits, rscale
 // f.rs[z]), one launch for all.
-template <int N1, int N2, int TI, int MODE, bool PAIR = false, bool F32OUT = false>
-__global__ void __launch_bounds__(kThreads) k_fft4(FftFields f, size_t es, size_t gs, int nrow,
+template <int N1, int N2, int TI, int NTH, int MODE, bool PAIR = false, bool F32OUT = false>
+__global__ void __launch_bounds__(NTH) k_fft4(FftFields f, size_t es, size_t gs, int nrow,
                                                    int act_nrc, const double2 *tw, const double2 *twh, double sg,
                                                    double scale, const double *r, int nr, int mlim,
                                                    int zin_lo, int zin_hi, int zout_lo, int zout_hi,
@@ -440,8 +440,8 @@ __global__ void __launch_bounds__(kThreads) k_fft4(FftFields f, size_t es, size_
     out = f.out[blockIdx.z];
     rscale = f.rs[blockIdx.z];
   }
-  constexpr int T1 = (TI * N2 + kThreads - 1) / kThreads;
-  constexpr int T2 = (TI * N1 + kThreads - 1) / kThreads;
+  constexpr int T1 = (TI * N2 + NTH - 1) / NTH;
+  constexpr int T2 = (TI * N1 + NTH - 1) / NTH;
   constexpr bool HALF = (MODE == 0 && N == 256);
   __shared__ double2 buf[HALF ? TI * N / 2 : TI * N];
   __shared__ double2 nyq[MODE == 2 ? TI : 1];
@@ -459,7 +459,7 @@ __global__ void __launch_bounds__(kThreads) k_fft4(FftFields f, size_t es, size_
   if (MODE == 2 && PAIR) {
     // stage 0 from radial pairs: tile rows l (x) and TH + l (nr - 1 - x)
     const float4 *pin = reinterpret_cast<const float4 *>(in);
-    for (int b = tid; b < TH * (N + 1); b += kThreads) {
+    for (int b = tid; b < TH * (N + 1); b += NTH) {
       const int l = b % TH, m = b / TH, x = i0 + l;
       float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
       // an ordinary load: the pairs were just written and are read from the cache
@@ -477,7 +477,7 @@ __global__ void __launch_bounds__(kThreads) k_fft4(FftFields f, size_t es, size_
     __syncthreads();
   } else if (MODE == 2) {
     // stage 0: C_m, m = 0..N, into LDS (C_N apart)
-    for (int b = tid; b < TI * (N + 1); b += kThreads) {
+    for (int b = tid; b < TI * (N + 1); b += NTH) {
       const int l = b % TI, m = b / TI, i = i0 + l;
       const double2 v = (i < rlim && m < mlim) ? ld_nt(&in[base + (size_t)m * es + i]) : make_double2(0.0, 0.0);
       if (m < N) buf[m * TI + l] = v;
@@ -490,7 +490,7 @@ __global__ void __launch_bounds__(kThreads) k_fft4(FftFields f, size_t es, size_
   double2 y1[T1][N1];
 #pragma unroll
   for (int t = 0; t < T1; ++t) {
-    const int b = tid + t * kThreads;
+    const int b = tid + t * NTH;
     if (b < TI * N2) {
       const int l = b % TI, n2 = b / TI, i = i0 + l;
       double2 v[N1];
@@ -538,7 +538,7 @@ __global__ void __launch_bounds__(kThreads) k_fft4(FftFields f, size_t es, size_
       if (h) __syncthreads();
 #pragma unroll
       for (int t = 0; t < T1; ++t) {
-        const int b = tid + t * kThreads;
+        const int b = tid + t * NTH;
         if (b < TI * N2) {
           const int l = b % TI, n2 = b / TI;
 #pragma unroll
@@ -548,7 +548,7 @@ __global__ void __launch_bounds__(kThreads) k_fft4(FftFields f, size_t es, size_
       __syncthreads();
 #pragma unroll
       for (int t = 0; t < T2; ++t) {
-        const int b = tid + t * kThreads;
+        const int b = tid + t * NTH;
         if (b < TI * N1) {
           const int l = b % TI, k1 = b / TI;
 #pragma unroll
@@ -561,11 +561,11 @@ __global__ void __launch_bounds__(kThreads) k_fft4(FftFields f, size_t es, size_
     }
 #pragma unroll
     for (int t = 0; t < T2; ++t)
-      if (tid + t * kThreads < TI * N1) dft_reg<N2>(y2[t], sg);
+      if (tid + t * NTH < TI * N1) dft_reg<N2>(y2[t], sg);
   } else {
 #pragma unroll
     for (int t = 0; t < T1; ++t) {
-      const int b = tid + t * kThreads;
+      const int b = tid + t * NTH;
       if (b < TI * N2) {
         const int l = b % TI, n2 = b / TI;
 #pragma unroll
@@ -577,7 +577,7 @@ __global__ void __launch_bounds__(kThreads) k_fft4(FftFields f, size_t es, size_
     // stage 2
 #pragma unroll
     for (int t = 0; t < T2; ++t) {
-      const int b = tid + t * kThreads;
+      const int b = tid + t * NTH;
       if (b < TI * N1) {
         const int l = b % TI, k1 = b / TI;
 #pragma unroll
@@ -589,7 +589,7 @@ __global__ void __launch_bounds__(kThreads) k_fft4(FftFields f, size_t es, size_
   if (MODE == 0 || MODE == 2) {
 #pragma unroll
     for (int t = 0; t < T2; ++t) {
-      const int b = tid + t * kThreads;
+      const int b = tid + t * NTH;
       if (b < TI * N1) {
         const int l = b % TI, k1 = b / TI;
         // the output row of tile row l (PAIR: pair x = i0 + l % TH)
@@ -621,7 +621,7 @@ __global__ void __launch_bounds__(kThreads) k_fft4(FftFields f, size_t es, size_
   __syncthreads();
 #pragma unroll
   for (int t = 0; t < T2; ++t) {
-    const int b = tid + t * kThreads;
+    const int b = tid + t * NTH;
     if (b < TI * N1) {
       const int l = b % TI, k1 = b / TI;
 #pragma unroll
@@ -629,7 +629,7 @@ __global__ void __launch_bounds__(kThreads) k_fft4(FftFields f, size_t es, size_
     }
   }
   __syncthreads();
-  for (int b = tid; b < TI * (N + 1); b += kThreads) {
+  for (int b = tid; b < TI * (N + 1); b += NTH) {
     const int l = b % TI, m = b / TI, i = i0 + l;
     const double2 zm = buf[(m % N) * TI + l];
     double2 zc = buf[((N - m) % N) * TI + l];
@@ -652,16 +652,16 @@ __global__ void __launch_bounds__(kThreads) k_fft4(FftFields f, size_t es, size_
 // i >= nr give zero products, as vector_product leaves them.
 // F32IN: the six velocity and vorticity fields are stored in FP32 at
 // f32_index (ub, the background flow, stays FP64).
-template <int N1, int N2, int TI, bool F32IN = false>
-__global__ void __launch_bounds__(kThreads) k_fft4_cross(double2 *o0, double2 *o1, double2 *o2, const double2 *v0,
+template <int N1, int N2, int TI, int NTH, bool F32IN = false>
+__global__ void __launch_bounds__(NTH) k_fft4_cross(double2 *o0, double2 *o1, double2 *o2, const double2 *v0,
                                                          const double2 *v1, const double2 *v2, const double2 *w0,
                                                          const double2 *w1, const double2 *w2, const double2 *ub,
                                                          size_t es, size_t gs, int nrow, const double2 *tw,
                                                          const double2 *twh, double scale, const double *r, int nr,
                                                          double *ln0, double *ln1, double *ln2, int mmax) {
   constexpr int N = N1 * N2;
-  constexpr int T1 = (TI * N2 + kThreads - 1) / kThreads;
-  constexpr int T2 = (TI * N1 + kThreads - 1) / kThreads;
+  constexpr int T1 = (TI * N2 + NTH - 1) / NTH;
+  constexpr int T2 = (TI * N1 + NTH - 1) / NTH;
   const double sg = -1.0;
   __shared__ double2 buf[TI * N];
   const int i0 = blockIdx.x * TI;
@@ -679,7 +679,7 @@ __global__ void __launch_bounds__(kThreads) k_fft4_cross(double2 *o0, double2 *o
   double2 y1[3][T1][N1];
 #pragma unroll
   for (int t = 0; t < T1; ++t) {
-    const int b = tid + t * kThreads;
+    const int b = tid + t * NTH;
     if (b < TI * N2) {
       const int l = b % TI, n2 = b / TI, i = i0 + l;
       double2 c0[N1], c1[N1], c2[N1];
@@ -745,7 +745,7 @@ __global__ void __launch_bounds__(kThreads) k_fft4_cross(double2 *o0, double2 *o
     if (comp > 0) __syncthreads();  // the previous component's untangling has read buf
 #pragma unroll
     for (int t = 0; t < T1; ++t) {
-      const int b = tid + t * kThreads;
+      const int b = tid + t * NTH;
       if (b < TI * N2) {
         const int l = b % TI, n2 = b / TI;
 #pragma unroll
@@ -756,7 +756,7 @@ __global__ void __launch_bounds__(kThreads) k_fft4_cross(double2 *o0, double2 *o
     double2 y2[T2][N2];
 #pragma unroll
     for (int t = 0; t < T2; ++t) {
-      const int b = tid + t * kThreads;
+      const int b = tid + t * NTH;
       if (b < TI * N1) {
         const int l = b % TI, k1 = b / TI;
 #pragma unroll
@@ -767,7 +767,7 @@ __global__ void __launch_bounds__(kThreads) k_fft4_cross(double2 *o0, double2 *o
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < T2; ++t) {
-      const int b = tid + t * kThreads;
+      const int b = tid + t * NTH;
       if (b < TI * N1) {
         const int l = b % TI, k1 = b / TI;
 #pragma unroll
@@ -776,7 +776,7 @@ __global__ void __launch_bounds__(kThreads) k_fft4_cross(double2 *o0, double2 *o
     }
     __syncthreads();
     // C_m = E + W^m O, m = 0..N, scaled 1/np
-    for (int b = tid; b < TI * (N + 1); b += kThreads) {
+    for (int b = tid; b < TI * (N + 1); b += NTH) {
       const int l = b % TI, m = b / TI, i = i0 + l;
       const double2 zm = buf[(m % N) * TI + l];
       double2 zc = buf[((N - m) % N) * TI + l];
@@ -846,6 +846,14 @@ __global__ void __launch_bounds__(kThreads) k_fftg_cross(CrossArgs a) {
   }
 }
 
+// Tiles of ti rows leave the card less than two workgroups to a CU: small
+// tiles (128 or 256 bytes of a line) then, each with the threads its items
+// need.  One slice of 128 x 128 is 4 workgroups of 32 rows: the fused product
+// takes 14.5 us there and 11.3 in tiles of 8, the phi transforms 8.2 and 7.1;
+// one slice of 256 x 256 15.9 against 15.1.  With two workgroups to a CU the
+// large tiles' longer lines are as fast or faster.
+bool few_tiles(int nrow, int ti, int nwg) { return (nrow + ti - 1) / ti * nwg < 512; }
+
 // grid_y: columns or planes (y) and fields (z) of the launch; false when N is
 // no length of the four-step kernels
 template <int MODE, bool PAIR = false, bool F32OUT = false>
@@ -853,25 +861,32 @@ bool launch_fft4(mlx_ctx *c, ProbeScope &ps, int N, dim3 grid_y, const FftFields
                  int act_nrc, const double2 *tw, const double2 *twh, double sg, double scale, int mlim = 1 << 30,
                  int zin_lo = 1, int zin_hi = 0, int zout_lo = 1, int zout_hi = 0, int pstride = 0) {
   const KitDev &k = c->kit;
-#define MLX_FFT4(N1_, N2_, TI_)                                                                                    \
+// NTH_ threads; small grids take TS_ rows a tile and TS_ max(N1, N2) threads
+#define MLX_FFT4_(N1_, N2_, TI_, NTH_)                                                                             \
   do {                                                                                                             \
     constexpr int TH_ = PAIR ? TI_ / 2 : TI_;                                                                      \
     dim3 grid((nrow + TH_ - 1) / TH_, grid_y.y, grid_y.z);                                                         \
-    probed_launch(ps, k_fft4<N1_, N2_, TI_, MODE, PAIR, F32OUT>, grid, dim3(kThreads), 0, c->stream, f, es, gs,   \
+    probed_launch(ps, k_fft4<N1_, N2_, TI_, NTH_, MODE, PAIR, F32OUT>, grid, dim3(NTH_), 0, c->stream, f, es, gs, \
                   nrow, act_nrc, tw, twh, sg, scale, k.r, k.nr, mlim, zin_lo, zin_hi, zout_lo, zout_hi, pstride);  \
     return true;                                                                                                   \
   } while (0)
+#define MLX_FFT4(N1_, N2_, TI_, TS_)                                                                               \
+  do {                                                                                                             \
+    if (few_tiles(PAIR ? 2 * nrow : nrow, TI_, grid_y.y * grid_y.z)) MLX_FFT4_(N1_, N2_, TS_, TS_ * N2_);          \
+    MLX_FFT4_(N1_, N2_, TI_, kThreads);                                                                            \
+  } while (0)
   switch (N) {
-    case 16: MLX_FFT4(4, 4, 64);
-    case 32: MLX_FFT4(4, 8, 64);
-    case 64: MLX_FFT4(8, 8, 32);
-    case 128: MLX_FFT4(8, 16, 16);
+    case 16: MLX_FFT4(4, 4, 64, 16);
+    case 32: MLX_FFT4(4, 8, 64, 8);
+    case 64: MLX_FFT4(8, 8, 32, 8);
+    case 128: MLX_FFT4(8, 16, 16, 8);
     case 256:
-      if (MODE == 0) MLX_FFT4(16, 16, 16);  // 64 KiB of LDS
-      MLX_FFT4(16, 16, 8);                  // the real modes also hold the Nyquist column
+      if (MODE == 0) MLX_FFT4_(16, 16, 16, kThreads);  // 64 KiB of LDS
+      MLX_FFT4_(16, 16, 8, kThreads);                  // the real modes also hold the Nyquist column
     default: return false;
   }
 #undef MLX_FFT4
+#undef MLX_FFT4_
 }
 
 // The groups of a plan: the two whose larger one is the smallest (the most
@@ -1023,24 +1038,32 @@ void fft_phi_cross(mlx_ctx *c, double2 *o0, double2 *o1, double2 *o2, const doub
   // fields written
   ProbeScope probe(c, MLX_PROBE_PHI_CROSS, k.nr * k.nz * ((f32in ? 48.0 : 96.0) * N + 16.0 * N + 48.0 * mmax),
                    3.0 * 2.5 * k.np * std::log2((double)k.np) * k.nr * k.nz + 18.0 * k.nr * k.np * k.nz);
-#define MLX_FFTX(N1_, N2_, TI_)                                                                                 \
+#define MLX_FFTX_(N1_, N2_, TI_, NTH_)                                                                          \
   do {                                                                                                          \
     dim3 grid((k.nrdim + TI_ - 1) / TI_, k.nzdim);                                                              \
     if (f32in)                                                                                                  \
-      probed_launch(probe, k_fft4_cross<N1_, N2_, TI_, true>, grid, dim3(kThreads), 0, c->stream, o0, o1, o2, v0,  \
+      probed_launch(probe, k_fft4_cross<N1_, N2_, TI_, NTH_, true>, grid, dim3(NTH_), 0, c->stream, o0, o1, o2, v0, \
                     v1, v2, w0, w1, w2, ub, (size_t)k.nrdim, plane, k.nrdim, k.tw_nph, k.tw_half, 1.0 / k.np, k.r, \
                     k.nr, ln0, ln1, ln2, mmax);                                                                 \
     else                                                                                                        \
-      probed_launch(probe, k_fft4_cross<N1_, N2_, TI_, false>, grid, dim3(kThreads), 0, c->stream, o0, o1, o2, v0, \
-                    v1, v2, w0, w1, w2, ub, (size_t)k.nrdim, plane, k.nrdim, k.tw_nph, k.tw_half, 1.0 / k.np, k.r, \
-                    k.nr, ln0, ln1, ln2, mmax);                                                                 \
+      probed_launch(probe, k_fft4_cross<N1_, N2_, TI_, NTH_, false>, grid, dim3(NTH_), 0, c->stream, o0, o1, o2, \
+                    v0, v1, v2, w0, w1, w2, ub, (size_t)k.nrdim, plane, k.nrdim, k.tw_nph, k.tw_half, 1.0 / k.np, \
+                    k.r, k.nr, ln0, ln1, ln2, mmax);                                                            \
+  } while (0)
+// a small tile of 32 points has the large one's thread pattern (one item each
+// in stage 2, none idle): the compiler then fuses the same products, and a
+// slice's result does not depend on the tile
+#define MLX_FFTX(N1_, N2_, TI_, TS_, NS_)                                                                       \
+  do {                                                                                                          \
+    if (few_tiles(k.nrdim, TI_, k.nzdim)) MLX_FFTX_(N1_, N2_, TS_, NS_);                                        \
+    else MLX_FFTX_(N1_, N2_, TI_, kThreads);                                                                    \
   } while (0)
   switch (N) {
-    case 16: MLX_FFTX(4, 4, 64); break;
-    case 32: MLX_FFTX(4, 8, 64); break;
-    case 64: MLX_FFTX(8, 8, 32); break;
-    case 128: MLX_FFTX(8, 16, 16); break;
-    case 256: MLX_FFTX(16, 16, 8); break;
+    case 16: MLX_FFTX(4, 4, 64, 16, 64); break;
+    case 32: MLX_FFTX(4, 8, 64, 16, 64); break;
+    case 64: MLX_FFTX(8, 8, 32, 8, 64); break;
+    case 128: MLX_FFTX(8, 16, 16, 8, 128); break;
+    case 256: MLX_FFTX_(16, 16, 8, kThreads); break;
     default: {
       CrossArgs a;
       a.g = groups_of(k.plan_nph, k.nrdim, 3 * k.nzdim);
@@ -1055,6 +1078,7 @@ void fft_phi_cross(mlx_ctx *c, double2 *o0, double2 *o1, double2 *o2, const doub
     }
   }
 #undef MLX_FFTX
+#undef MLX_FFTX_
   HIPCHK(hipGetLastError());
 }
 
