@@ -562,7 +562,9 @@ void v2t_f64(mlx_ctx *c, hipStream_t s, const double2 *ur, const double2 *up, co
   g.nzc = k.chopzl, g.nzcu = k.chopzu, g.zlo = zlo, g.zhi = zhi, g.mbeg = mbeg, g.mend = mend;
   g.tpitch = k.mfma_ap, g.ksplit = ksplit, g.zso = zso, g.kstride = kstride;
   // eight waves and 32 slices where that leaves two workgroups to a CU, four
-  // waves (32 rows a) and 16 slices below (150 x 120 x 90: 76 against 49 us)
+  // waves (32 rows a) and 8 slices below (150 x 120 x 90: 76 against 51 us; one
+  // slice, 256 x 256: 37 us in tiles of 16 slices, 25 in tiles of 8, one accumulator
+  // block a wave; 128 x 128: 16.0 and 12.3)
   g.nyt = (k.nzdim + 31) / 32, g.nsp = (M + 63) / 64;
   const int ncol = (mend < npc ? mend : npc) - mbeg;
   if (ksplit > 1) {
@@ -572,8 +574,8 @@ void v2t_f64(mlx_ctx *c, hipStream_t s, const double2 *ur, const double2 *up, co
   } else if (ncol * g.nyt * g.nsp >= 512) {
     hipLaunchKernelGGL((k_v2t_f64m<8, 32, false>), dim3((mend - mbeg) * g.nyt * g.nsp * ksplit), dim3(512), 0, s, g);
   } else {
-    g.nyt = (k.nzdim + 15) / 16, g.nsp = (M + 31) / 32;
-    hipLaunchKernelGGL((k_v2t_f64m<4, 16, false>), dim3((mend - mbeg) * g.nyt * g.nsp * ksplit), dim3(256), 0, s, g);
+    g.nyt = (k.nzdim + 7) / 8, g.nsp = (M + 31) / 32;
+    hipLaunchKernelGGL((k_v2t_f64m<4, 8, false>), dim3((mend - mbeg) * g.nyt * g.nsp * ksplit), dim3(256), 0, s, g);
   }
   HIPCHK(hipGetLastError());
 }
