@@ -139,7 +139,8 @@ class Scalar:
             self.h = h
             self._owned = True
             if space != 'PPP':
-                self.set_meta(space=space)
+                # a new field's ln and offsets are zero: nothing to read back
+                tfm._check(self.lib.mlx_field_set_meta(tfm.ctx, h, space.encode(), 0.0, (ctypes.c_int32 * 3)(0, 0, 0)))
         else:
             self.h = handle
             self._owned = False

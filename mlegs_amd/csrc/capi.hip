@@ -29,34 +29,45 @@ void need_kit(mlx_ctx *c) {
   if (!c->kit.ready) MLX_THROW(MLX_E_ARG, "transformation kit is not initialized");
 }
 
+// Under capture nothing may be allocated or freed, a kept block no more than a
+// new one: hipMalloc and hipFree refuse there.
 mlx_field *field_new(mlx_ctx *c) {
+  const size_t ne = sizeof(double2) * c->nelem, ns = sizeof(double) * 8;
+  const bool cap = capturing(c);
   mlx_field *f = new mlx_field();
-  if (hipMalloc(&f->e, sizeof(double2) * c->nelem) != hipSuccess) {
+  if (cap) {
+    if (hipMalloc(&f->e, ne) == hipSuccess && hipMalloc(&f->sc, ns) != hipSuccess) (void)hipFree(f->e);
+  } else {
+    f->e = static_cast<double2 *>(field_mem_get(c->device, ne));
+    if (f->e && !(f->sc = static_cast<double *>(field_mem_get(c->device, ns)))) field_mem_put(c->device, f->e, ne);
+  }
+  if (!f->sc) {
     delete f;
     MLX_THROW(MLX_E_ALLOC, "scalar_init: device allocation failed");
   }
-  if (hipMalloc(&f->sc, sizeof(double) * 8) != hipSuccess) {
-    (void)hipFree(f->e);
-    delete f;
-    MLX_THROW(MLX_E_ALLOC, "scalar_init: device allocation failed");
-  }
-  HIPCHK(hipMemsetAsync(f->e, 0, sizeof(double2) * c->nelem, c->stream));
-  HIPCHK(hipMemsetAsync(f->sc, 0, sizeof(double) * 8, c->stream));
+  k_zero_field(c, f->e, f->sc);
   return f;
 }
 
-void field_free(mlx_field *f) {
+void field_free(mlx_ctx *c, mlx_field *f) {
   if (!f) return;
-  if (f->e) (void)hipFree(f->e);
-  if (f->sc) (void)hipFree(f->sc);
+  field_mem_put(c->device, f->e, sizeof(double2) * c->nelem);
+  field_mem_put(c->device, f->sc, sizeof(double) * 8);
   delete f;
 }
 
-// deep copy (mlegs_scalar_init.f90:106-140)
+// deep copy (mlegs_scalar_init.f90:106-140): data and ln in one launch, where two
+// copies are two launches and more host time each (a 32 x 16 x 8 round trip of the
+// transforms 36.7 us with them, 32.6 without); at 256^3, where launches
+// do not count, the runtime's copy is 2 of 42 us faster
 void fcopy(mlx_ctx *c, mlx_field *d, const mlx_field *s) {
   if (d == s) return;
-  HIPCHK(hipMemcpyAsync(d->e, s->e, sizeof(double2) * c->nelem, hipMemcpyDeviceToDevice, c->stream));
-  HIPCHK(hipMemcpyAsync(d->sc, s->sc, sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+  if (sizeof(double2) * c->nelem < ((size_t)64 << 20)) {
+    k_copy_field(c, d->e, s->e, d->sc, s->sc);
+  } else {
+    HIPCHK(hipMemcpyAsync(d->e, s->e, sizeof(double2) * c->nelem, hipMemcpyDeviceToDevice, c->stream));
+    HIPCHK(hipMemcpyAsync(d->sc, s->sc, sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+  }
   std::memcpy(d->space, s->space, 4);
   std::memcpy(d->off, s->off, sizeof(d->off));
 }
@@ -1160,16 +1171,17 @@ int mlx_ctx_create(const mlx_params *p, int device, void *stream, mlx_ctx **out)
       HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
       c->own_stream = true;
     }
-    HIPCHK(hipMalloc(&c->dsmall, sizeof(double) * 4096));
+    HIPCHK(dev_malloc(&c->dsmall, sizeof(double) * 4096));
     HIPCHK(hipMemsetAsync(c->dsmall, 0, sizeof(double) * 4096, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
-    HIPCHK(hipMalloc(&c->dpart, sizeof(double) * kPartMax));
+    HIPCHK(dev_malloc(&c->dpart, sizeof(double) * kPartMax));
     HIPCHK(hipHostMalloc(&c->hsmall, sizeof(double) * 4096));
   });
   if (rc != MLX_OK) {
     delete c;
     return rc;
   }
+  field_mem_contexts(device, 1);
   *out = c;
   return MLX_OK;
 }
@@ -1178,8 +1190,9 @@ int mlx_ctx_destroy(mlx_ctx *c) {
   if (!c) return MLX_OK;
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
-  for (mlx_field *f : c->pool) field_free(f);
+  for (mlx_field *f : c->pool) field_free(c, f);
   c->pool.clear();
+  field_mem_contexts(c->device, -1);
   lu_cache_free(c);
   hyp_cache_free(c);
   for (auto &v : c->probe.ev)
@@ -1244,7 +1257,7 @@ int mlx_kit_init(mlx_ctx *c) {
     }
     for (double2 *&s : c->scr) {
       if (s) (void)hipFree(s);
-      if (hipMalloc(&s, sizeof(double2) * c->nelem) != hipSuccess) MLX_THROW(MLX_E_ALLOC, "scratch allocation failed");
+      if (dev_malloc(&s, sizeof(double2) * c->nelem) != hipSuccess) MLX_THROW(MLX_E_ALLOC, "scratch allocation failed");
       HIPCHK(hipMemsetAsync(s, 0, sizeof(double2) * c->nelem, c->stream));
     }
   });
@@ -1309,8 +1322,8 @@ int mlx_field_create(mlx_ctx *c, mlx_field **out) {
 
 int mlx_field_destroy(mlx_ctx *c, mlx_field *f) {
   return guarded(c, [&] {
-    HIPCHK(hipStreamSynchronize(c->stream));
-    field_free(f);
+    if (capturing(c)) HIPCHK(hipStreamSynchronize(c->stream));  // refused there
+    field_free(c, f);
   });
 }
 
@@ -1744,12 +1757,12 @@ int mlx_vortex_create(mlx_ctx *c, const mlx_field *psi, const mlx_field *chi, co
       fcopy(c, v->f[1], chi);
       for (int i = 2; i < 8; ++i) set_space(v->f[i], "FFF");
       fcopy(c, v->f[8], uz);
-      HIPCHK(hipMalloc(&v->gains, sizeof(double) * 2));
-      HIPCHK(hipMalloc(&v->flag, sizeof(int)));
+      HIPCHK(dev_malloc(&v->gains, sizeof(double) * 2));
+      HIPCHK(dev_malloc(&v->flag, sizeof(int)));
       HIPCHK(hipMemsetAsync(v->gains, 0, sizeof(double) * 2, c->stream));
       HIPCHK(hipMemsetAsync(v->flag, 0, sizeof(int), c->stream));
     } catch (...) {
-      for (mlx_field *f : v->f) field_free(f);
+      for (mlx_field *f : v->f) field_free(c, f);
       delete v;
       throw;
     }
@@ -1761,7 +1774,7 @@ int mlx_vortex_destroy(mlx_ctx *c, mlx_vortex *v) {
   return guarded(c, [&] {
     if (!v) return;
     HIPCHK(hipStreamSynchronize(c->stream));
-    for (mlx_field *f : v->f) field_free(f);
+    for (mlx_field *f : v->f) field_free(c, f);
     if (v->gains) (void)hipFree(v->gains);
     if (v->flag) (void)hipFree(v->flag);
     delete v;

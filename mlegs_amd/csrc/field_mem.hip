@@ -1,0 +1,112 @@
+// Device memory of fields, kept between one field's end and the next one's
+// start.
+//
+// hipFree waits for the whole device and unmaps, hipMalloc maps: about 110 and
+// 20 us for a field, with the GPU idle meanwhile.  Code that makes copies as it
+// goes paid that for each: a gradient of twelve steps at 128 x 64 x 64 frees
+// 120 blocks, 13 of its 24 ms.
+//
+// A freed block waits in `limbo` until a hipFree has passed, whose implicit wait
+// for the device covers the work of every stream that was issued before the
+// block was given up, the caller's own streams included; only then is it handed
+// out again.  32 blocks in limbo are enough for one such hipFree (of the
+// smallest of them).  What is kept is bounded per device (kMaxBytes, kMaxBlocks;
+// a block over kMaxBlock is freed at once), is returned when an allocation of
+// this library finds no memory, and when the device's last context ends.
+// Blocks are matched by size alone, under a mutex: no owner, stream or address
+// plays a part.
+#include <mutex>
+
+#include "mlx_internal.h"
+
+namespace {
+
+constexpr size_t kMaxBytes = (size_t)2 << 30;
+constexpr size_t kMaxBlock = kMaxBytes / 8;
+constexpr size_t kMaxBlocks = 256, kLimbo = 32;
+
+struct Block {
+  void *p;
+  size_t bytes;
+};
+struct Pool {
+  std::vector<Block> limbo, ready;
+  size_t bytes = 0;  // of both
+  int contexts = 0;
+
+  void drop(Block b) {
+    (void)hipFree(b.p);
+    bytes -= b.bytes;
+  }
+  void release() {
+    for (auto *v : {&limbo, &ready}) {
+      for (const Block &b : *v) drop(b);
+      v->clear();
+    }
+  }
+};
+
+std::mutex g_mutex;
+std::map<int, Pool> &pools() {
+  static auto *p = new std::map<int, Pool>;  // outlives every static destructor
+  return *p;
+}
+
+}  // namespace
+
+namespace mlx {
+
+void *field_mem_get(int device, size_t bytes) {
+  {
+    std::lock_guard<std::mutex> lock(g_mutex);
+    Pool &q = pools()[device];
+    for (size_t i = q.ready.size(); i-- > 0;)
+      if (q.ready[i].bytes == bytes) {
+        void *p = q.ready[i].p;
+        q.ready[i] = q.ready.back();
+        q.ready.pop_back();
+        q.bytes -= bytes;
+        return p;
+      }
+  }
+  void *p = nullptr;
+  return dev_malloc(&p, bytes) == hipSuccess ? p : nullptr;
+}
+
+void field_mem_put(int device, void *p, size_t bytes) {
+  if (!p) return;
+  std::lock_guard<std::mutex> lock(g_mutex);
+  Pool &q = pools()[device];
+  if (q.contexts <= 0 || bytes > kMaxBlock || q.bytes + bytes > kMaxBytes || q.limbo.size() + q.ready.size() >= kMaxBlocks) {
+    (void)hipFree(p);
+  } else {
+    q.limbo.push_back({p, bytes});
+    q.bytes += bytes;
+    if (q.limbo.size() < kLimbo) return;
+    size_t least = 0;
+    for (size_t i = 1; i < q.limbo.size(); ++i)
+      if (q.limbo[i].bytes < q.limbo[least].bytes) least = i;
+    q.drop(q.limbo[least]);
+    q.limbo.erase(q.limbo.begin() + least);
+  }
+  // the hipFree has waited for all work on the device
+  q.ready.insert(q.ready.end(), q.limbo.begin(), q.limbo.end());
+  q.limbo.clear();
+}
+
+bool field_mem_release(int device) {
+  std::lock_guard<std::mutex> lock(g_mutex);
+  Pool &q = pools()[device];
+  const bool any = q.bytes > 0;
+  q.release();
+  return any;
+}
+
+void field_mem_contexts(int device, int d) {
+  std::lock_guard<std::mutex> lock(g_mutex);
+  Pool &q = pools()[device];
+  q.contexts += d;
+  if (q.contexts <= 0) q.release();
+}
+
+}  // namespace mlx

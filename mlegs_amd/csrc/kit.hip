@@ -202,7 +202,7 @@ double2 *upload_twiddles(int n, int count, double denom) {
     h[t].y = (double)sinl(a);
   }
   double2 *d = nullptr;
-  HIPCHK(hipMalloc(&d, sizeof(double2) * h.size()));
+  HIPCHK(dev_malloc(&d, sizeof(double2) * h.size()));
   HIPCHK(hipMemcpy(d, h.data(), sizeof(double2) * h.size(), hipMemcpyHostToDevice));
   (void)n;
   return d;
@@ -212,7 +212,7 @@ template <class T>
 T *dalloc(size_t n) {
   T *p = nullptr;
   if (n == 0) n = 1;
-  if (hipMalloc(&p, n * sizeof(T)) != hipSuccess) MLX_THROW(MLX_E_ALLOC, "kit: device allocation failed");
+  if (dev_malloc(&p, n * sizeof(T)) != hipSuccess) MLX_THROW(MLX_E_ALLOC, "kit: device allocation failed");
   return p;
 }
 

@@ -312,7 +312,7 @@ const WorkTable &get_work(mlx_ctx *c, int kind, int nroff) {
   WorkTable wt;
   wt.n = (int)h.size();
   if (wt.n > 0) {
-    HIPCHK(hipMalloc(&wt.d, sizeof(int4) * h.size()));
+    HIPCHK(dev_malloc(&wt.d, sizeof(int4) * h.size()));
     HIPCHK(hipMemcpy(wt.d, h.data(), sizeof(int4) * h.size(), hipMemcpyHostToDevice));
   }
   c->work[key] = wt;

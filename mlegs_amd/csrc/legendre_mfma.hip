@@ -701,7 +701,7 @@ void mfma_tables(mlx_ctx *c) {
   k.mfma_ap = AP;
   auto alloc = [&](auto *&p) {
     if (p) (void)hipFree(p);
-    if (hipMalloc(&p, sizeof(*p) * n) != hipSuccess) MLX_THROW(MLX_E_ALLOC, "kit: table allocation failed");
+    if (dev_malloc(&p, sizeof(*p) * n) != hipSuccess) MLX_THROW(MLX_E_ALLOC, "kit: table allocation failed");
   };
   alloc(k.pfg32);
   alloc(k.tVg32);

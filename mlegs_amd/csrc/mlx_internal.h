@@ -185,16 +185,42 @@ struct mlx_ctx {
   double2 *v2t_part = nullptr;
 };
 
+// Device memory of fields (field_mem.hip): blocks given up are handed out again
+// once the device has finished what was issued before.
+namespace mlx {
+void *field_mem_get(int device, size_t bytes);  // nullptr: no memory
+void field_mem_put(int device, void *p, size_t bytes);
+bool field_mem_release(int device);             // whether anything was held
+void field_mem_contexts(int device, int d);     // a context begins (+1), ends (-1)
+}  // namespace mlx
+
+// hipMalloc; kept field memory is returned first where there is none left
+template <class T>
+hipError_t dev_malloc(T **p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  int device = 0;
+  if (e == hipErrorOutOfMemory && hipGetDevice(&device) == hipSuccess && mlx::field_mem_release(device)) {
+    (void)hipGetLastError();
+    e = hipMalloc(p, bytes);
+  }
+  return e;
+}
+
+// whether c's stream is recording a graph
+inline bool capturing(const mlx_ctx *c) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  HIPCHK(hipStreamIsCapturing(c->stream, &st));
+  return st != hipStreamCaptureStatusNone;
+}
+
 // A buffer the context allocates on first use (*p of bytes).  Under stream
 // capture nothing may be allocated: a step run once before the capture
 // allocates it.
 inline void lazy_alloc(mlx_ctx *c, void **p, size_t bytes, const char *what) {
   if (*p) return;
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  HIPCHK(hipStreamIsCapturing(c->stream, &st));
-  if (st != hipStreamCaptureStatusNone)
+  if (capturing(c))
     MLX_THROW(MLX_E_ARG, std::string(what) + ": first use under stream capture (run one step before capturing)");
-  if (hipMalloc(p, bytes) != hipSuccess) {
+  if (dev_malloc(p, bytes) != hipSuccess) {
     *p = nullptr;
     MLX_THROW(MLX_E_ALLOC, std::string(what) + ": allocation failed");
   }
@@ -423,7 +449,8 @@ void k_idel2_preln00(mlx_ctx *c, double2 *e, double *ln, double preln, int nroff
 void k_axpby(mlx_ctx *c, double2 *dst, double *dln, double a, const double2 *src, const double *sln, double b);
 void k_read_field(mlx_ctx *c, const double2 *src, double *part);
 void k_write_field(mlx_ctx *c, double2 *dst, double v);
-void k_copy_field(mlx_ctx *c, double2 *dst, const double2 *src);
+void k_copy_field(mlx_ctx *c, double2 *dst, const double2 *src, double *dln = nullptr, const double *sln = nullptr);
+void k_zero_field(mlx_ctx *c, double2 *dst, double *sc);  // data and the 8 device scalars
 void k_abcn_rhs(mlx_ctx *c, double2 *sh, double *shln, const double2 *s, const double *sln,
                 const double2 *nl, const double *nlln, const double2 *nlp, const double *nlpln,
                 const double2 *svis, double dt, double a, int ab2);

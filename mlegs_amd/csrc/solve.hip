@@ -569,11 +569,11 @@ LuCache &lu_get(mlx_ctx *c, double alpha, int kind, int nroff) {
     if (e.pvw) (void)hipFree(e.pvw);
     if (e.anyp) (void)hipFree(e.anyp);
   };
-  if (hipMalloc(&fac, sizeof(double) * nsys * k.nrdim * LDAB) != hipSuccess ||
-      hipMalloc(&piv, nsys * k.nrdim) != hipSuccess ||
-      hipMalloc(&e.sol, sizeof(double) * 7 * nrows) != hipSuccess ||
-      hipMalloc(&e.pvw, sizeof(uint64_t) * nsys * NSEG) != hipSuccess ||
-      hipMalloc(&e.anyp, sizeof(int) * nsys) != hipSuccess) {
+  if (dev_malloc(&fac, sizeof(double) * nsys * k.nrdim * LDAB) != hipSuccess ||
+      dev_malloc(&piv, nsys * k.nrdim) != hipSuccess ||
+      dev_malloc(&e.sol, sizeof(double) * 7 * nrows) != hipSuccess ||
+      dev_malloc(&e.pvw, sizeof(uint64_t) * nsys * NSEG) != hipSuccess ||
+      dev_malloc(&e.anyp, sizeof(int) * nsys) != hipSuccess) {
     cleanup();
     MLX_THROW(MLX_E_ALLOC, "ihelm: cannot allocate LU factors");
   }

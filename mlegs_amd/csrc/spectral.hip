@@ -1381,9 +1381,18 @@ __global__ void k_sum_parts(const double *part, int nb, double *out) {
 }
 
 // plain copy of a whole field (also the known-size reference for HBM counters)
-__global__ void k_copy_field_(double2 *__restrict__ d, const double2 *__restrict__ s, size_t n) {
+__global__ void k_copy_field_(double2 *__restrict__ d, const double2 *__restrict__ s, size_t n, double *dln,
+                              const double *sln) {
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
     d[i] = s[i];
+  if (dln && blockIdx.x == 0 && threadIdx.x == 0) dln[0] = sln[0];
+}
+
+// a new field: data and device scalars in one launch
+__global__ void k_zero_field_(double2 *__restrict__ d, size_t n, double *sc) {
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
+    d[i] = make_double2(0.0, 0.0);
+  if (blockIdx.x == 0 && threadIdx.x < 8) sc[threadIdx.x] = 0.0;
 }
 
 // read-only and write-only passes over a whole field (the HBM ceilings of a
@@ -1602,9 +1611,9 @@ HypLu &hyp_get(mlx_ctx *c, int power, double alpha, double beta, int nroff, int 
   h.nsys = k.npchop * ((h.nkk + 31) / 32) * 32;  // blocks of 32 systems
   const int LDAB = 3 * power + 1;
   // factor rows of 3P + 2 doubles (HypLu's layout)
-  if (hipMalloc(&h.ab, sizeof(double) * (size_t)nrc * (LDAB + 1) * h.nsys) != hipSuccess ||
-      hipMalloc(&h.pv, (size_t)nrc * h.nsys) != hipSuccess ||
-      hipMalloc(&h.sink, sizeof(double2) * 64 * hyp_sink_rows(nrc, power)) != hipSuccess) {
+  if (dev_malloc(&h.ab, sizeof(double) * (size_t)nrc * (LDAB + 1) * h.nsys) != hipSuccess ||
+      dev_malloc(&h.pv, (size_t)nrc * h.nsys) != hipSuccess ||
+      dev_malloc(&h.sink, sizeof(double2) * 64 * hyp_sink_rows(nrc, power)) != hipSuccess) {
     hyp_free(h);
     MLX_THROW(MLX_E_ALLOC, "ihelmp: cannot allocate the banded factors");
   }
@@ -1696,8 +1705,12 @@ void k_write_field(mlx_ctx *c, double2 *dst, double v) {
   hipLaunchKernelGGL(k_write_field_, dim3(grid_for(c->nelem)), dim3(kT), 0, c->stream, dst, c->nelem, v);
 }
 
-void k_copy_field(mlx_ctx *c, double2 *dst, const double2 *src) {
-  hipLaunchKernelGGL(k_copy_field_, dim3(grid_for(c->nelem)), dim3(kT), 0, c->stream, dst, src, c->nelem);
+void k_copy_field(mlx_ctx *c, double2 *dst, const double2 *src, double *dln, const double *sln) {
+  hipLaunchKernelGGL(k_copy_field_, dim3(grid_for(c->nelem)), dim3(kT), 0, c->stream, dst, src, c->nelem, dln, sln);
+}
+
+void k_zero_field(mlx_ctx *c, double2 *dst, double *sc) {
+  hipLaunchKernelGGL(k_zero_field_, dim3(grid_for(c->nelem)), dim3(kT), 0, c->stream, dst, c->nelem, sc);
 }
 
 void k_abcn_rhs(mlx_ctx *c, double2 *sh, double *shln, const double2 *s, const double *sln, const double2 *nl,
