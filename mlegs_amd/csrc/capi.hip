@@ -236,15 +236,18 @@ struct DealiasLimits {
 
 // dl (the time loop, which de-aliases f right after): the systems of the
 // modes de-aliasing zeroes are not solved
-void ihelmp(mlx_ctx *c, mlx_field *f, int power, double alpha, double beta, const DealiasLimits *dl = nullptr) {
+// f2: a second field of f's radial offset, solved with it
+void ihelmp(mlx_ctx *c, mlx_field *f, int power, double alpha, double beta, const DealiasLimits *dl = nullptr,
+            mlx_field *f2 = nullptr) {
   need_kit(c);
   check_power("ihelmp", power);
   to_fff(c, f);
+  if (f2) to_fff(c, f2);
   if (std::fabs(alpha) < 5e-14)
     MLX_THROW(MLX_E_ARG, "ihelmp: alpha equals to zero. Inversion of 0*identity is impossible");
   const bool lim = dl && dl->on;
   k_ihelmp(c, f->e, f->sc, power, alpha, beta, f->off[0], sing_flag(c), lim ? dl->pcut : -1, lim ? dl->zlo : 1,
-           lim ? dl->zhi : 0);
+           lim ? dl->zhi : 0, f2 ? f2->e : nullptr, f2 ? f2->sc : nullptr);
 }
 
 // fftreat (mlegs_scalar_ops.f90:1002-1063): far-field smoothing.  delsqp
@@ -289,9 +292,11 @@ void check_step_inputs(mlx_ctx *c, std::initializer_list<const mlx_field *> fs) 
 // hypervisc del^p as g (del^p + b del2), g = hypervisc (-1)^(p/2+1),
 // b = visc / g, inverted by ihelmp with alpha = -1/(dt g) (febe) or
 // -2/(dt g) (abcn, whose right-hand side adds dt/2 g helmp(s, p, 0, b))
-// dl: as abcn's (the time loop de-aliases s right after)
+// dl: as abcn's (the time loop de-aliases s right after); t, nlt, nlt_p: a second
+// field's step (abcn only, s's radial offset), solved with the first
 void step_hyper(mlx_ctx *c, mlx_field *s, const mlx_field *nl, const mlx_field *nl_p, double dt,
-                const DealiasLimits *dl = nullptr) {
+                const DealiasLimits *dl = nullptr, mlx_field *t = nullptr, const mlx_field *nlt = nullptr,
+                const mlx_field *nlt_p = nullptr) {
   const int pw = c->p.hyperpow;
   const double g = c->p.hypervisc * (((pw / 2 + 1) % 2) ? -1.0 : 1.0);
   const double b = c->p.visc / g;
@@ -299,9 +304,13 @@ void step_hyper(mlx_ctx *c, mlx_field *s, const mlx_field *nl, const mlx_field *
     // helmp(s, pw, 0, b) and the right-hand side in one column pass
     const double a = -2.0 / (dt * g);
     const bool lim = dl && dl->on;
-    k_abcn_rhs_hyp(c, s->e, s->sc, nl->e, nl->sc, nl_p->e, nl_p->sc, dt, a, g, b, pw, s->off[0],
-                   lim ? dl->pcut : -1, lim ? dl->zlo : 1, lim ? dl->zhi : 0, lim);
-    ihelmp(c, s, pw, a, b, dl);
+    auto rhs = [&](mlx_field *f, const mlx_field *n, const mlx_field *n_p) {
+      k_abcn_rhs_hyp(c, f->e, f->sc, n->e, n->sc, n_p->e, n_p->sc, dt, a, g, b, pw, f->off[0], lim ? dl->pcut : -1,
+                     lim ? dl->zlo : 1, lim ? dl->zhi : 0, lim);
+    };
+    rhs(s, nl, nl_p);
+    if (t) rhs(t, nlt, nlt_p);
+    ihelmp(c, s, pw, a, b, dl, t);
   } else {
     const double a = -1.0 / (dt * g);
     k_abcn_rhs_g(c, s->e, s->sc, s->e, s->sc, nl->e, nl->sc, nullptr, nullptr, nullptr, dt, a, 0, g);
@@ -445,12 +454,18 @@ void abcn(mlx_ctx *c, mlx_field *s, mlx_field *s_p, mlx_field *nl, mlx_field *nl
 // same factors, read once for both fields)
 void abcn_pair(mlx_ctx *c, mlx_field *s1, mlx_field *s1p, mlx_field *nl1, mlx_field *nl1p, mlx_field *s2,
                mlx_field *s2p, mlx_field *nl2, mlx_field *nl2p, double dt, const DealiasLimits &dl) {
-  if (!dl.on || s1->off[0] != s2->off[0] || c->p.hyperpow != 0) {
+  if (s1->off[0] != s2->off[0] || (!dl.on && c->p.hyperpow == 0)) {
     abcn(c, s1, s1p, nl1, nl1p, dt, false, true, &dl);
     abcn(c, s2, s2p, nl2, nl2p, dt, false, true, &dl);
     return;
   }
   check_step_inputs(c, {s1, nl1, s1p, nl1p, s2, nl2, s2p, nl2p});
+  if (c->p.hyperpow != 0) {
+    step_hyper(c, s1, nl1, nl1p, dt, &dl, s2, nl2, nl2p);
+    fmove(nl1p, nl1);
+    fmove(nl2p, nl2);
+    return;
+  }
   if (c->p.visc < 5e-14) MLX_THROW(MLX_E_ARG, "abcn: inviscid case and no linear term in rhs. semi-implicit time adv is impossible");
   const double a = -2.0 / (dt * c->p.visc);
   if (std::fabs(a) < 5e-14) MLX_THROW(MLX_E_ARG, "ihelm: alpha equals to zero. Inversion of 0*identity is impossible");

@@ -107,9 +107,9 @@ struct LuCache {
 // i = kk % 32; nsys counts the blocks' slots); entry r of row j of a
 // system's LAPACK band storage (LDAB = 3P + 1 entries: U's diagonal and 2P
 // superdiagonals at r = 2P - q, L's P multipliers at r = 2P + 1 ..) at
-// ab[((j * nblk + b) * (3P + 2) + r') * 32 + i], r' = r (r <= 2P) or r + 1:
-// the 32 systems of a block are adjacent for every entry; the row
-// interchange of row j as the offset to the pivot row at
+// ab[(j * nblk + b) * (3P + 2) * 32 + (r' / 2) * 64 + 2 i + r' % 2], r' = r
+// (r <= 2P) or r + 1: two entries a 16-byte load, the 32 systems of a block
+// adjacent for every pair; the row interchange of row j as the offset to the pivot row at
 // pv[(j * nblk + b) * 32 + i].
 struct HypLu {
   int power = 0;
@@ -411,9 +411,10 @@ void k_abcn_rhs_g(mlx_ctx *c, double2 *sh, double *shln, const double2 *s, const
 // factors kept per (power, alpha, beta, nroff); a factorization that meets a
 // zero pivot sets *sing (device int) to 1 and throws before anything is solved
 // pcut > 0: only columns m < pcut are solved; slices zlo..zhi are not solved
-// (their right-hand sides are zero or are zeroed afterwards)
+// (their right-hand sides are zero or are zeroed afterwards); e2, sln2: a second
+// field solved in the same launch
 void k_ihelmp(mlx_ctx *c, double2 *e, double *sln, int power, double alpha, double beta, int nroff, int *sing,
-              int pcut = -1, int zlo = 1, int zhi = 0);
+              int pcut = -1, int zlo = 1, int zhi = 0, double2 *e2 = nullptr, double *sln2 = nullptr);
 // fftreat's physical-space step on the PFF lines of columns m < npc
 void k_fftreat_mid(mlx_ctx *c, double2 *e, int npc);
 void k_chop(mlx_ctx *c, double2 *e, const char *space, int nroff);

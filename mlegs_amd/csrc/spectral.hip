@@ -1049,19 +1049,21 @@ __global__ void __launch_bounds__(256) k_ihelmp_fac_(double *__restrict__ ab, in
   constexpr int ROW = 3 * P + 2;
   for (int q = tid; q < LDAB * nn; q += blockDim.x) {
     const int j = q / LDAB, r = q % LDAB;
-    ab[(((size_t)j * nblk + blk) * ROW + (r <= KV ? r : r + 1)) * 32 + ib] = AB[q];
+    const int t = r <= KV ? r : r + 1;
+    ab[((size_t)j * nblk + blk) * ROW * 32 + (t / 2) * 64 + 2 * ib + t % 2] = AB[q];
   }
   for (int j = tid; j < nn; j += blockDim.x) pv[((size_t)j * nblk + blk) * 32 + ib] = (int8_t)piv[j];
 }
 
 // The (0,0) column's log term before the solve (the reference's bl, bl2):
 // lnp = ln / alpha; b(:, 0, 0) -= leg_del2(0, ak_0)^(Q-1) bl2 + beta bl2,
-// with bl2 the log term's Laplacian rows; ln <- lnp.  One workgroup.
+// with bl2 the log term's Laplacian rows; ln <- lnp.  A workgroup per field.
 template <int P>
-__global__ void __launch_bounds__(256) k_ihelmp_ln_(double2 *e, double *sln, const double *d2c, const double *ak,
-                                                    const double *lognorm, double alpha, double beta, int ne, int nn,
-                                                    double ell) {
+__global__ void __launch_bounds__(256) k_ihelmp_ln_(double2 *e, double *sln, double2 *e2, double *sln2,
+                                                    const double *d2c, const double *ak, const double *lognorm,
+                                                    double alpha, double beta, int ne, int nn, double ell) {
   constexpr int Q = P / 2;
+  if (blockIdx.x == 1) e = e2, sln = sln2;
   extern __shared__ double hsm[];
   double *v = hsm, *t = hsm + nn;
   const int tid = threadIdx.x;
@@ -1096,13 +1098,24 @@ __global__ void __launch_bounds__(256) k_ihelmp_ln_(double2 *e, double *sln, con
   if (tid == 0) sln[0] = lnp;
 }
 
-// gbtrs on the kept factors.  A 64-lane workgroup owns column m and 32
-// consecutive |kappa| values; lanes 2i and 2i + 1 solve slices kk and
-// nz - kk of system kk (they read the same factor entries).  Each lane runs
-// the two sweeps over its own column in registers, in the reference's order
-// of operations: the forward sweep keeps rows j .. j + P (interchange, then
+// gbtrs on the kept factors, for NF fields of the same operator.  The factors
+// are real, so the real and the imaginary part of a column are two independent
+// systems: every lane owns one part of one column.  A 64-lane workgroup owns
+// column m and 16 / NF consecutive |kappa| values; the 4 NF lanes of a system
+// (slices kk and nz - kk, the fields, the parts) read the same factor entries.
+// Each lane runs the two sweeps in registers, in the reference's order of
+// operations: the forward sweep keeps rows j .. j + P (interchange, then
 // the P eliminations of row j), the back substitution the 2P pending rows
-// above row j (x_j, then its 2P updates).  The factor entries of the rows
+// above row j (x_j, then its 2P updates).
+// What bounds it is the chain of rows of one wave (a few hundred waves: about one
+// to a CU): 60 to 120 instructions issue one after another per row,
+// so the work per lane counts and not the factors' bytes.  Both parts on a lane and
+// a launch a field took 239 us a field at 256 x 128 x 128, P = 8 (2 x 239 of a
+// step's 1140 us); a part a lane and both fields in one launch 196 us for the
+// two, the factors read once; two factor entries a load, selects left out where
+// stored zeros do the same, and loads kept in row order 171.  Deeper rings
+// (RF, RB up to 16, 8) measure the same.
+// The factor entries of the rows
 // ahead are loaded RF (forward) and RB (back) rows early.  The loops have no
 // branches around loads or stores, so the loads stay in flight across rows:
 // rows past the system's end run with zero multipliers and no interchange
@@ -1111,159 +1124,152 @@ __global__ void __launch_bounds__(256) k_ihelmp_ln_(double2 *e, double *sln, con
 // (its slice chopped, the twin of a self-conjugate slice, past the last
 // |kappa|) works in `sink` (garbage in, garbage out, never read as data).
 // A slice visited twice by the chop (z_count 2) is solved twice.
-template <int P>
-__global__ void __launch_bounds__(64) k_ihelmp_sol_(double2 *e, const double *__restrict__ ab,
+constexpr int kHypRF = 4, kHypRB = 4;
+
+template <int P, int NF>
+__global__ void __launch_bounds__(64) k_ihelmp_sol_(double2 *e, double2 *e2, const double *__restrict__ ab,
                                                     const int8_t *__restrict__ pv, double2 *sink, int nrdim,
                                                     int npdim, int nz, int nrc, int npc, int nkk, int nzc, int nzcu,
                                                     int zlo, int zhi) {
-  constexpr int KV = 2 * P, ROW = 3 * P + 2, RF = 4, RB = 2;
+  constexpr int KV = 2 * P, ROW = 3 * P + 2, RF = kHypRF, RB = kHypRB, SYS = 16 / NF;
   const int m = blockIdx.y, lane = threadIdx.x;
   const int nn = nrcs_dev(nrc, npc, m);  // uniform over the workgroup
   if (nn <= 0) return;
-  const int kk0 = blockIdx.x * 32 + lane / 2, twin = lane & 1;
+  const int part = lane & 1, twin = (lane / (2 * NF)) & 1;
+  const int kk0 = blockIdx.x * SYS + lane / (4 * NF);
+  if (NF == 2 && (lane & 2)) e = e2;
   const bool have = kk0 < nkk;
   const int kk = have ? kk0 : 0;
   const int k = twin ? (nz - kk) % nz : kk;
   const bool valid = have && (!twin || (kk != 0 && 2 * kk != nz));
   // slices zlo..zhi are left as they are
   const int cnt = (valid && !(k >= zlo && k <= zhi)) ? z_count(k, nzc, nzcu) : 0;
-  // HypLu's block of the workgroup's 32 systems, the lane's place in it
-  const size_t nblk = (size_t)npc * ((nkk + 31) / 32), blk = (size_t)m * ((nkk + 31) / 32) + blockIdx.x;
-  const int ib = lane / 2;
-  double2 *const colv = e + (size_t)k * nrdim * npdim + (size_t)nrdim * m;
-  double2 *const snk = sink + (size_t)lane * (nrc + KV + RF);  // rows j < nrc + RF written, -KV-1.. read
-  const double2 z2 = make_double2(0.0, 0.0);
-  // row j's factors (clamped to the system's rows): entry r at rw[32 r]
+  // HypLu's block of 32 systems, the lane's place in it (SYS divides 32)
+  const size_t nblk = (size_t)npc * ((nkk + 31) / 32), blk = (size_t)m * ((nkk + 31) / 32) + blockIdx.x * SYS / 32;
+  const int ib = kk0 % 32;
+  // row i of a column at [2 i]
+  double *const colv = reinterpret_cast<double *>(e + (size_t)k * nrdim * npdim + (size_t)nrdim * m) + part;
+  // rows j < nrc + RF written, -KV-1.. read
+  double *const snk = reinterpret_cast<double *>(sink + (size_t)lane * (nrc + KV + RF)) + part;
+  // row j's factors (clamped to the system's rows): entries 2 t and 2 t + 1 at rw[32 t]
 #define MLX_JC(j) ((j) < 0 ? 0 : ((j) > nn - 1 ? nn - 1 : (j)))
-#define MLX_ROW(j) (ab + ((size_t)MLX_JC(j) * nblk + blk) * ROW * 32 + ib)
+#define MLX_ROW(j) (reinterpret_cast<const double2 *>(ab + ((size_t)MLX_JC(j) * nblk + blk) * ROW * 32) + ib)
   // a right-hand-side entry (zero outside 0 .. nn - 1), read without a branch
-  // (component selects: a select of whole double2 values becomes a select of
-  // addresses)
 #define MLX_IDX(i) (((i) >= 0 && (i) < nn) ? (i) : 0)
 #define MLX_IN(i) ((i) >= 0 && (i) < nn)
-#define MLX_ZSEL(dst, in, v)      \
-  do {                            \
-    const bool in_ = (in);        \
-    dst.x = in_ ? (v).x : 0.0;    \
-    dst.y = in_ ? (v).y : 0.0;    \
-  } while (0)
-  // ring slot u: the raw entries of row j (loads only: the row-validity
-  // selects are applied where the values are used, so no instruction waits
-  // on a load before its row comes up)
+  // ring slot u: the entries of row j.  The scheduling barriers after each row keep
+  // its loads in the order of the rows, so that a row waits for its own only
 #define MLX_LOAD_F(j, u)                                                            \
   do {                                                                              \
-    const double *rw = MLX_ROW(j) + (KV + 2) * 32;                                  \
-    _Pragma("unroll") for (int q = 0; q < P; ++q) L[u][q] = rw[32 * q];             \
+    const double2 *rw = MLX_ROW(j) + (P + 1) * 32;                                  \
+    _Pragma("unroll") for (int q = 0; q < P / 2; ++q) L[u][q] = rw[32 * q];         \
     jp[u] = pv[((size_t)MLX_JC(j) * nblk + blk) * 32 + ib];                         \
-    nb[u] = col[MLX_IDX((j) + P + 1)];                                              \
+    nb[u] = col[2 * MLX_IDX((j) + P + 1)];                                          \
   } while (0)
 #define MLX_LOAD_B(j, u)                                                            \
   do {                                                                              \
-    const double *rw = MLX_ROW(j);                                                  \
-    _Pragma("unroll") for (int q = 0; q <= KV; ++q) U[u][q] = rw[32 * (KV - q)];    \
-    yb[u] = col[MLX_IDX((j) - KV - 1)];                                             \
+    const double2 *rw = MLX_ROW(j);                                                 \
+    _Pragma("unroll") for (int q = 0; q <= P; ++q) U[u][q] = rw[32 * q];            \
+    yb[u] = col[2 * MLX_IDX((j) - KV - 1)];                                         \
   } while (0)
 #pragma unroll 1
   for (int rep = 0; rep < 2; ++rep) {
     if (!__any(rep < cnt)) break;
     // the lane's working column: its slice, or the sink
-    double2 *const col = (rep < cnt) ? colv : snk + KV + 1;
+    double *const col = (rep < cnt) ? colv : snk + 2 * (KV + 1);
     // forward sweep over rows 0 .. nn - 1 (and padding to a multiple of RF):
     // F[q] = b(j + q); row j stores y_j
     {
-      double L[RF][P];
+      double2 L[RF][P / 2];
       int jp[RF];
-      double2 nb[RF];  // b(j + P + 1) for the rows ahead
-      double2 F[P + 1];
+      double nb[RF];  // b(j + P + 1) for the rows ahead
+      double F[P + 1];
 #pragma unroll
       for (int q = 0; q <= P; ++q) {
-        const double2 v = col[MLX_IDX(q)];
-        MLX_ZSEL(F[q], MLX_IN(q), v);
+        const double v = col[2 * MLX_IDX(q)];
+        F[q] = MLX_IN(q) ? v : 0.0;
       }
 #pragma unroll
-      for (int u = 0; u < RF; ++u) MLX_LOAD_F(u, u);
+      for (int u = 0; u < RF; ++u) {
+        MLX_LOAD_F(u, u);
+        __builtin_amdgcn_sched_barrier(0);
+      }
 #pragma unroll 1
       for (int j0 = 0; j0 < nn; j0 += RF) {
 #pragma unroll
         for (int u = 0; u < RF; ++u) {
           const int j = j0 + u;
-          // interchange rows j and j + jp, as selects over the window: the
-          // empty asm hides that the mask has one bit, so the compiler keeps
-          // F in registers instead of indexing it through memory; component
-          // selects, since a select of whole double2 values becomes a select
-          // of addresses
-          const bool el = j < nn - 1;  // row j has eliminations
-          unsigned pm = 1u << (el ? jp[u] : 0);
-          asm volatile("" : "+v"(pm));
-          double f0x = F[0].x, f0y = F[0].y;
+          // interchange rows j and j + jp (no lane has one in most rows), as
+          // selects over the window: the empty asm hides that the mask has
+          // one bit, so the compiler keeps F in registers instead of indexing
+          // it through memory
+          const int jr = j < nn - 1 ? jp[u] : 0;
+          if (__any(jr)) {
+            unsigned pm = 1u << jr;
+            asm volatile("" : "+v"(pm));
+            double f0 = F[0];
 #pragma unroll
-          for (int q = 1; q <= P; ++q) {
-            const bool sw = (pm >> q) & 1u;
-            const double ax = F[q].x, ay = F[q].y;
-            F[q].x = sw ? F[0].x : ax;
-            F[q].y = sw ? F[0].y : ay;
-            f0x = sw ? ax : f0x;
-            f0y = sw ? ay : f0y;
+            for (int q = 1; q <= P; ++q) {
+              const bool sw = (pm >> q) & 1u;
+              const double a = F[q];
+              F[q] = sw ? F[0] : a;
+              f0 = sw ? a : f0;
+            }
+            F[0] = f0;
           }
-          F[0].x = f0x;
-          F[0].y = f0y;
-          // multipliers of rows below nn - 1 are stored zeros
+          // multipliers of rows below nn - 1, row nn - 1's own and those read for
+          // the rows past it are stored zeros
 #pragma unroll
-          for (int q = 1; q <= P; ++q) {
-            const double l = el ? L[u][q - 1] : 0.0;
-            F[q].x -= l * F[0].x;
-            F[q].y -= l * F[0].y;
-          }
-          double2 *const o = (j < nn) ? col + j : snk + j;
+          for (int q = 1; q <= P; ++q) F[q] -= (q % 2 ? L[u][(q - 1) / 2].x : L[u][(q - 1) / 2].y) * F[0];
+          double *const o = (j < nn) ? col + 2 * j : snk + 2 * j;
           *o = F[0];
 #pragma unroll
           for (int q = 0; q < P; ++q) F[q] = F[q + 1];
-          MLX_ZSEL(F[P], MLX_IN(j + P + 1), nb[u]);
+          F[P] = MLX_IN(j + P + 1) ? nb[u] : 0.0;
           MLX_LOAD_F(j + RF, u);
+          __builtin_amdgcn_sched_barrier(0);
         }
       }
     }
     // back substitution over rows nn - 1 .. 0 (and padding): B[q] = b(j - q),
     // pending; row j stores x_j
     {
-      double U[RB][KV + 1];
-      double2 yb[RB];  // b(j - 2P - 1) for the rows ahead
-      double2 B[KV + 1];
+      double2 U[RB][P + 1];
+      double yb[RB];  // b(j - 2P - 1) for the rows ahead
+      double B[KV + 1];
 #pragma unroll
       for (int q = 0; q <= KV; ++q) {
-        const double2 v = col[MLX_IDX(nn - 1 - q)];
-        MLX_ZSEL(B[q], MLX_IN(nn - 1 - q), v);
+        const double v = col[2 * MLX_IDX(nn - 1 - q)];
+        B[q] = MLX_IN(nn - 1 - q) ? v : 0.0;
       }
 #pragma unroll
-      for (int u = 0; u < RB; ++u) MLX_LOAD_B(nn - 1 - u, u);
+      for (int u = 0; u < RB; ++u) {
+        MLX_LOAD_B(nn - 1 - u, u);
+        __builtin_amdgcn_sched_barrier(0);
+      }
 #pragma unroll 1
       for (int j0 = nn - 1; j0 >= 0; j0 -= RB) {
 #pragma unroll
         for (int u = 0; u < RB; ++u) {
           const int j = j0 - u;
-          const bool el = j >= 0;  // a row of the system
-          const double d = el ? U[u][0] : 1.0;
-          const double2 x = make_double2(B[0].x / d, B[0].y / d);
-          double2 *const o = (j >= 0) ? col + j : snk + (j + KV + 1);
+          const double x = B[0] / U[u][P].x;
+          double *const o = (j >= 0) ? col + 2 * j : snk + 2 * (j + KV + 1);
           *o = x;
-          // U(j - q, j) of rows above the first is a stored zero
+          // U(j - q, j) of rows above the first is a stored zero (rows past the
+          // system's end only pass values on to each other)
 #pragma unroll
-          for (int q = 1; q <= KV; ++q) {
-            const double a = el ? U[u][q] : 0.0;
-            B[q].x -= a * x.x;
-            B[q].y -= a * x.y;
-          }
+          for (int q = 1; q <= KV; ++q) B[q] -= (q % 2 ? U[u][(KV - q) / 2].y : U[u][(KV - q) / 2].x) * x;
 #pragma unroll
           for (int q = 0; q < KV; ++q) B[q] = B[q + 1];
-          MLX_ZSEL(B[KV], MLX_IN(j - KV - 1), yb[u]);
+          B[KV] = MLX_IN(j - KV - 1) ? yb[u] : 0.0;
           MLX_LOAD_B(j - RB, u);
+          __builtin_amdgcn_sched_barrier(0);
         }
       }
     }
   }
 #undef MLX_LOAD_B
 #undef MLX_LOAD_F
-#undef MLX_ZSEL
 #undef MLX_IN
 #undef MLX_IDX
 #undef MLX_ROW
@@ -1578,8 +1584,8 @@ void hyp_free(HypLu &h) {
   h.sink = nullptr;
 }
 
-// rows of the solve's sink per lane (k_ihelmp_sol_: nrc + 2P + 4)
-size_t hyp_sink_rows(int nrc, int power) { return (size_t)nrc + 2 * power + 4; }
+// rows of the solve's sink per lane (k_ihelmp_sol_: nrc + 2P + RF)
+size_t hyp_sink_rows(int nrc, int power) { return (size_t)nrc + 2 * power + kHypRF; }
 
 // The factors for (power, alpha, beta, nroff): kept ones, else factored now
 // (a zero pivot throws, nothing is kept)
@@ -1648,7 +1654,7 @@ void hyp_cache_free(mlx_ctx *c) {
 }
 
 void k_ihelmp(mlx_ctx *c, double2 *e, double *sln, int power, double alpha, double beta, int nroff, int *sing,
-              int pcut, int zlo, int zhi) {
+              int pcut, int zlo, int zhi, double2 *e2, double *sln2) {
   const KitDev &k = c->kit;
   const int nrc = k.nrchop + nroff;
   // chop_index's check (mlegs_scalar_ops.f90:2053): the rows of a system lie
@@ -1660,14 +1666,18 @@ void k_ihelmp(mlx_ctx *c, double2 *e, double *sln, int power, double alpha, doub
   if (nrc <= 0) return;
   HypLu &h = hyp_get(c, power, alpha, beta, nroff, nrc, sing);
   const int npc_grid = (pcut > 0 && pcut < k.npchop) ? pcut : k.npchop;
-  dim3 grid((h.nkk + 31) / 32, npc_grid);
-#define MLX_IHS(P_)                                                                                             \
-  do {                                                                                                          \
-    hipLaunchKernelGGL(k_ihelmp_ln_<P_>, dim3(1), dim3(256), 2 * sizeof(double) * nrc, c->stream, e, sln, k.d2c, \
-                       k.ak, k.lognorm, alpha, beta, k.ne, nrc, k.ell);                                        \
-    hipLaunchKernelGGL(k_ihelmp_sol_<P_>, grid, dim3(64), 0, c->stream, e, h.ab, h.pv, h.sink, k.nrdim, k.npdim, \
-                       k.nzdim, \
-                       nrc, k.npchop, h.nkk, k.chopzl, k.chopzu, zlo, zhi);                                    \
+#define MLX_IHS(P_)                                                                                                \
+  do {                                                                                                             \
+    hipLaunchKernelGGL(k_ihelmp_ln_<P_>, dim3(e2 ? 2 : 1), dim3(256), 2 * sizeof(double) * nrc, c->stream, e, sln, \
+                       e2, sln2, k.d2c, k.ak, k.lognorm, alpha, beta, k.ne, nrc, k.ell);                           \
+    if (e2)                                                                                                        \
+      hipLaunchKernelGGL((k_ihelmp_sol_<P_, 2>), dim3((h.nkk + 7) / 8, npc_grid), dim3(64), 0, c->stream, e, e2,   \
+                         h.ab, h.pv, h.sink, k.nrdim, k.npdim, k.nzdim, nrc, k.npchop, h.nkk, k.chopzl, k.chopzu,  \
+                         zlo, zhi);                                                                                \
+    else                                                                                                           \
+      hipLaunchKernelGGL((k_ihelmp_sol_<P_, 1>), dim3((h.nkk + 15) / 16, npc_grid), dim3(64), 0, c->stream, e, e,  \
+                         h.ab, h.pv, h.sink, k.nrdim, k.npdim, k.nzdim, nrc, k.npchop, h.nkk, k.chopzl, k.chopzu,  \
+                         zlo, zhi);                                                                                \
   } while (0)
   switch (power) {
     case 4: MLX_IHS(4); break;
