@@ -320,7 +320,7 @@ __global__ void __launch_bounds__(512) k_leg_bwd_f64m(LegFields f, LegDims d, co
 // limits): the even and odd waves share the six folds of the three fields (a
 // workgroup of one parity read and folded all three for itself), the tables go
 // from L2 into the registers of the wave that uses them, and the rows leave in
-// whole columns: 387 -> 311 us.  One tile of 16 rows a wave: two would need 320
+// whole columns: 387 -> 282 us.  One tile of 16 rows a wave: two would need 320
 // accumulator registers.
 // Only rows < nrchop - m are computed: the three rows of the radial offset are
 // chopped afterwards by the reference.  Columns mbeg .. mend - 1.
@@ -337,9 +337,14 @@ struct V2tArgs {
   int nrdim, npdim, nz, nr, nrh, nrc, npc, nzc, nzcu, nyt, nsp, zlo, zhi, mbeg, mend, tpitch, ksplit;
   size_t zso, kstride;
 };
-template <int NW, int KT, bool COL0>
-__global__ void __launch_bounds__(64 * NW) k_v2t_f64m(V2tArgs g) {
-  constexpr int NTH = 64 * NW, NT = KT / 8, XC = 8, KS = XC / 4, PC = 2 * KT + 2, PL = XC * PC, NB = 6 * PL;
+// Four waves (32 rows a, both parities) and 8 slices a workgroup for every size, held
+// to the registers of four workgroups a CU: at 256^3 282 us, where eight waves and
+// 32 slices (half the table and field reads from L2, one workgroup to a CU) take
+// 316, 16 slices 321, and this tile without the bound 320.  150 x 120 x 90: 51 us
+// against 76 with eight waves; one slice, 256 x 256: 25 against 37 with 16 slices.
+template <bool COL0>
+__global__ void __launch_bounds__(256, 4) k_v2t_f64m(V2tArgs g) {
+  constexpr int NW = 4, KT = 8, NTH = 64 * NW, NT = KT / 8, XC = 8, KS = XC / 4, PC = 2 * KT + 2, PL = XC * PC, NB = 6 * PL;
   constexpr int NP = NW / 2, R = 16 * NW, SPR = R + 1;  // output rows, their LDS pitch
   constexpr int NF = (XC * KT + NTH - 1) / NTH;
   constexpr int NLDS = 2 * NB > 16 * SPR ? 2 * NB : 16 * SPR;
@@ -561,21 +566,13 @@ void v2t_f64(mlx_ctx *c, hipStream_t s, const double2 *ur, const double2 *up, co
   g.nrdim = k.nrdim, g.npdim = k.npdim, g.nz = k.nzdim, g.nr = k.nr, g.nrh = k.nrh, g.nrc = k.nrchop, g.npc = npc;
   g.nzc = k.chopzl, g.nzcu = k.chopzu, g.zlo = zlo, g.zhi = zhi, g.mbeg = mbeg, g.mend = mend;
   g.tpitch = k.mfma_ap, g.ksplit = ksplit, g.zso = zso, g.kstride = kstride;
-  // eight waves and 32 slices where that leaves two workgroups to a CU, four
-  // waves (32 rows a) and 8 slices below (150 x 120 x 90: 76 against 51 us; one
-  // slice, 256 x 256: 37 us in tiles of 16 slices, 25 in tiles of 8, one accumulator
-  // block a wave; 128 x 128: 16.0 and 12.3)
-  g.nyt = (k.nzdim + 31) / 32, g.nsp = (M + 63) / 64;
-  const int ncol = (mend < npc ? mend : npc) - mbeg;
+  g.nyt = (k.nzdim + 7) / 8, g.nsp = (M + 31) / 32;
+  const dim3 grid((mend - mbeg) * g.nyt * g.nsp * ksplit);
   if (ksplit > 1) {
     if (mbeg != 0 || mend != 1) MLX_THROW(MLX_E_ARG, "vec2tp: radial shares of column 0 only");
-    g.nyt = (k.nzdim + 15) / 16, g.nsp = (M + 31) / 32;
-    hipLaunchKernelGGL((k_v2t_f64m<4, 16, true>), dim3(g.nyt * g.nsp * ksplit), dim3(256), 0, s, g);
-  } else if (ncol * g.nyt * g.nsp >= 512) {
-    hipLaunchKernelGGL((k_v2t_f64m<8, 32, false>), dim3((mend - mbeg) * g.nyt * g.nsp * ksplit), dim3(512), 0, s, g);
+    hipLaunchKernelGGL(k_v2t_f64m<true>, grid, dim3(256), 0, s, g);
   } else {
-    g.nyt = (k.nzdim + 7) / 8, g.nsp = (M + 31) / 32;
-    hipLaunchKernelGGL((k_v2t_f64m<4, 8, false>), dim3((mend - mbeg) * g.nyt * g.nsp * ksplit), dim3(256), 0, s, g);
+    hipLaunchKernelGGL(k_v2t_f64m<false>, grid, dim3(256), 0, s, g);
   }
   HIPCHK(hipGetLastError());
 }
