@@ -56,6 +56,11 @@ void field_free(mlx_ctx *c, mlx_field *f) {
   delete f;
 }
 
+void fmeta(mlx_field *d, const mlx_field *s) {
+  std::memcpy(d->space, s->space, 4);
+  std::memcpy(d->off, s->off, sizeof(d->off));
+}
+
 // deep copy (mlegs_scalar_init.f90:106-140): data and ln in one launch, where two
 // copies are two launches and more host time each (a 32 x 16 x 8 round trip of the
 // transforms 36.7 us with them, 32.6 without); at 256^3, where launches
@@ -68,8 +73,7 @@ void fcopy(mlx_ctx *c, mlx_field *d, const mlx_field *s) {
     HIPCHK(hipMemcpyAsync(d->e, s->e, sizeof(double2) * c->nelem, hipMemcpyDeviceToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(d->sc, s->sc, sizeof(double), hipMemcpyDeviceToDevice, c->stream));
   }
-  std::memcpy(d->space, s->space, 4);
-  std::memcpy(d->off, s->off, sizeof(d->off));
+  fmeta(d, s);
 }
 
 // dst takes src's data (buffers are exchanged; src becomes scratch)
@@ -434,18 +438,16 @@ void abcn(mlx_ctx *c, mlx_field *s, mlx_field *s_p, mlx_field *nl, mlx_field *nl
   if (c->p.visc < 5e-14) MLX_THROW(MLX_E_ARG, "abcn: inviscid case and no linear term in rhs. semi-implicit time adv is impossible");
   double a = -2.0 / (dt * c->p.visc);
   const bool lim = dl && dl->on;
-  if (lim && std::fabs(a) < 5e-14)
+  if (std::fabs(a) < 5e-14)
     MLX_THROW(MLX_E_ARG, "ihelm: alpha equals to zero. Inversion of 0*identity is impossible");
-  // lim: ihelm's log-term step rides on the log-coefficient update
-  k_abcn_rhs_d2(c, s->e, s->sc, nl->e, nl->sc, nl_p->e, nl_p->sc, dt, a, s->off[0], lim ? dl->pcut : -1,
-                lim ? dl->zlo : 1, lim ? dl->zhi : 0, lim);
-  if (lim) {
-    k_helm_solve(c, s->e, a, 0, s->off[0], dl->pcut, dl->zlo, dl->zhi);
-  } else {
-    ihelm(c, s, a);
-  }
+  // nl_p <- nl rides on the right-hand side where no field is given twice
+  const bool keep = !lim && !swap_nl && nl_p != nl && nl_p != s && nl_p != s_p && nl != s && nl != s_p;
+  const AbcnRhs f = {s->e, s->sc, nl->e, nl->sc, nl_p->e, nl_p->sc};
+  k_abcn_rhs_d2(c, &f, 1, dt, a, s->off[0], lim ? dl->pcut : -1, lim ? dl->zlo : 1, lim ? dl->zhi : 0, lim, keep);
+  k_helm_solve(c, s->e, a, 0, s->off[0], lim ? dl->pcut : -1, lim ? dl->zlo : 1, lim ? dl->zhi : 0);
   if (copy_prev) fcopy(c, s_p, s);
   if (swap_nl) fmove(nl_p, nl);
+  else if (keep) fmeta(nl_p, nl);
   else fcopy(c, nl_p, nl);
 }
 
@@ -469,10 +471,9 @@ void abcn_pair(mlx_ctx *c, mlx_field *s1, mlx_field *s1p, mlx_field *nl1, mlx_fi
   if (c->p.visc < 5e-14) MLX_THROW(MLX_E_ARG, "abcn: inviscid case and no linear term in rhs. semi-implicit time adv is impossible");
   const double a = -2.0 / (dt * c->p.visc);
   if (std::fabs(a) < 5e-14) MLX_THROW(MLX_E_ARG, "ihelm: alpha equals to zero. Inversion of 0*identity is impossible");
-  k_abcn_rhs_d2(c, s1->e, s1->sc, nl1->e, nl1->sc, nl1p->e, nl1p->sc, dt, a, s1->off[0], dl.pcut, dl.zlo, dl.zhi,
-                true);
-  k_abcn_rhs_d2(c, s2->e, s2->sc, nl2->e, nl2->sc, nl2p->e, nl2p->sc, dt, a, s2->off[0], dl.pcut, dl.zlo, dl.zhi,
-                true);
+  const AbcnRhs f[2] = {{s1->e, s1->sc, nl1->e, nl1->sc, nl1p->e, nl1p->sc},
+                        {s2->e, s2->sc, nl2->e, nl2->sc, nl2p->e, nl2p->sc}};
+  k_abcn_rhs_d2(c, f, 2, dt, a, s1->off[0], dl.pcut, dl.zlo, dl.zhi, true, false);
   k_helm_solve(c, s1->e, a, 0, s1->off[0], dl.pcut, dl.zlo, dl.zhi, s2->e);
   fmove(nl1p, nl1);
   fmove(nl2p, nl2);

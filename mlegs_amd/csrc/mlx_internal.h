@@ -455,11 +455,20 @@ void k_zero_field(mlx_ctx *c, double2 *dst, double *sc);  // data and the 8 devi
 void k_abcn_rhs(mlx_ctx *c, double2 *sh, double *shln, const double2 *s, const double *sln,
                 const double2 *nl, const double *nlln, const double2 *nlp, const double *nlpln,
                 const double2 *svis, double dt, double a, int ab2);
-// abcn's right-hand side in place on e (= s), with svis = del2(s) formed per column
-void k_abcn_rhs_d2(mlx_ctx *c, double2 *e, double *ln, const double2 *nl, const double *nlln, const double2 *nlp,
-                   const double *nlpln, double dt, double a, int nroff, int pcut = -1,
-                   int zlo = 1, int zhi = 0,
-                   bool helm_pre = false);
+// abcn's right-hand sides in place on e (= s) of nf (1 or 2) fields, with svis =
+// del2(s) formed per column, and ihelm's log-term step.  act: s, N and N_p are chopped,
+// only the active rows are read and written; keep (whole fields, not with act):
+// N_p <- N, data and ln
+struct AbcnRhs {
+  double2 *e;
+  double *ln;
+  const double2 *nl;
+  const double *nlln;
+  double2 *nlp;
+  double *nlpln;
+};
+void k_abcn_rhs_d2(mlx_ctx *c, const AbcnRhs *f, int nf, double dt, double a, int nroff, int pcut, int zlo, int zhi,
+                   bool act, bool keep);
 // abcn's hyperviscous right-hand side in place on e (= s), with svis =
 // helmp(s, power, 0, b) formed per column; act: s, N, N_p chopped (rows past
 // the system's rows zero), only the active rows read and written

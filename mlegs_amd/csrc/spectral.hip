@@ -476,17 +476,25 @@ __device__ inline void band_pow(double2 *y, const double2 *x, double2 *tmp, int 
 // where del2 acts on the rows of s's radial offset (applied as often as the
 // kk-loops visit the slice, log-term correction of (0,0) after) and leaves
 // every other entry equal to s, as the reference's copy-then-del2 does.
-// pre (nlln, nlpln given): k_abcn_ln_ followed by ihelm's log-term step
+// act: k_abcn_ln_ followed by ihelm's log-term step
 // (k_helm_pre_ with alpha = a), in the (0,0) workgroup: ln <- a (ln + dt
 // (1.5 nl.ln - 0.5 nl_p.ln)) / a, and rows 0..2 of the (0,0) column lose the
 // log term's Laplacian.  No other workgroup reads ln.
-__global__ void __launch_bounds__(256) k_abcn_rhs_d2_(double2 *e, double *sln, const double2 *nl,
-                                                      const double2 *nlp, const double *d2c, const double *lognorm,
-                                                      const double *ak, int nrdim, int npdim, int ne, int nrc,
-                                                      int npc, int nzc, int nzcu, double ell, double dt, double a,
-                                                      double visc, int pcut, int zlo, int zhi, const double *nlln,
-                                                      const double *nlpln, int act) {
+// keep: N's copy into N_p rides on the pass that reads both (the whole field is
+// visited then): abcn at 256 x 128 x 128 77.5 -> 75.8 us.  blockIdx.z: psi and chi of
+// the time loop in one launch (5.0 us each in launches of their own at
+// 128 x 128 x 1).
+__global__ void __launch_bounds__(256) k_abcn_rhs_d2_(mlx::AbcnRhs f0, mlx::AbcnRhs f1, const double *d2c,
+                                                      const double *lognorm, const double *ak, int nrdim, int npdim,
+                                                      int ne, int nrc, int npc, int nzc, int nzcu, double ell,
+                                                      double dt, double a, double visc, int pcut, int zlo, int zhi,
+                                                      int act, int keep) {
   extern __shared__ double2 lds[];
+  const mlx::AbcnRhs f = blockIdx.z ? f1 : f0;
+  double2 *const e = f.e, *const nlp = f.nlp;
+  double *const sln = f.ln;
+  const double2 *const nl = f.nl;
+  const double *const nlln = act ? f.nlln : nullptr, *const nlpln = f.nlpln;
   double2 *S = lds, *V = lds + nrdim, *T = lds + 2 * nrdim;
   const int m = blockIdx.x, k = blockIdx.y;
   // columns m >= pcut and slices zlo..zhi: left as they are (the caller
@@ -532,6 +540,7 @@ __global__ void __launch_bounds__(256) k_abcn_rhs_d2_(double2 *e, double *sln, c
       if (i == 2) o.x -= 2.0 / 3.0 / ell2 / exp(lognorm[2]) * l;
     }
     e[off + i] = o;
+    if (keep) nlp[off + i] = y;
   }
   if (pre) {
     __syncthreads();  // every read of sln above is done
@@ -599,6 +608,19 @@ __global__ void __launch_bounds__(256) k_abcn_rhs_hyp_(double2 *e, const double 
 __global__ void k_abcn_ln_(double *shln, const double *sln, const double *nlln, const double *nlpln, double dt,
                            double a) {
   shln[0] = a * (sln[0] + dt * (1.5 * nlln[0] - 0.5 * nlpln[0]));
+}
+
+// the same followed by ihelm's log-term step (k_helm_pre_) on the right-hand
+// side e and (keep) by nl_p.ln <- nl.ln: the order and roundings of the three steps
+__global__ void k_abcn_ln_pre_(mlx::AbcnRhs f, const double *lognorm, double dt, double a, double ell, int keep) {
+  const double sh = a * (f.ln[0] + dt * (1.5 * f.nlln[0] - 0.5 * f.nlpln[0]));
+  const double l = sh / a;
+  f.ln[0] = l;
+  const double ell2 = ell * ell;
+  f.e[0].x -= 4.0 / 3.0 / ell2 / exp(lognorm[0]) * l;
+  f.e[1].x += 2.0 / 1.0 / ell2 / exp(lognorm[1]) * l;
+  f.e[2].x -= 2.0 / 3.0 / ell2 / exp(lognorm[2]) * l;
+  if (keep) f.nlpln[0] = f.nlln[0];
 }
 
 __global__ void k_scale_rows_(double2 *e, const double *r, int nr, int nrdim, int npdim, int nz, int inverse) {
@@ -1739,24 +1761,27 @@ void k_abcn_rhs_g(mlx_ctx *c, double2 *sh, double *shln, const double2 *s, const
                      nlpln, svis, dt, a, g, ab2, c->nelem);
 }
 
-void k_abcn_rhs_d2(mlx_ctx *c, double2 *e, double *ln, const double2 *nl, const double *nlln, const double2 *nlp,
-                   const double *nlpln, double dt, double a, int nroff, int pcut, int zlo, int zhi, bool helm_pre) {
+void k_abcn_rhs_d2(mlx_ctx *c, const AbcnRhs *f, int nf, double dt, double a, int nroff, int pcut, int zlo, int zhi,
+                   bool act, bool keep) {
   const KitDev &k = c->kit;
   const int nrc = k.nrchop + nroff;
   if (nrc > k.nrdim_ref) MLX_THROW(MLX_E_ARG, "chop_index: chopping in r too large");
   if (pcut <= 0 || pcut > k.npdim) pcut = k.npdim;
-  if (helm_pre && zlo <= 0 && zhi >= 0) MLX_THROW(MLX_E_ARG, "abcn: the (0,0) column must be in the solved range");
-  dim3 grid(pcut, k.nzdim);
+  if (act && zlo <= 0 && zhi >= 0) MLX_THROW(MLX_E_ARG, "abcn: the (0,0) column must be in the solved range");
+  dim3 grid(pcut, k.nzdim, nf);
   size_t lds = 3 * sizeof(double2) * (size_t)k.nrdim;
-  // the log coefficient first: the data kernel reads s's ln for the (0,0) correction
-  // with helm_pre the (0,0) workgroup also takes ihelm's log-term step
+  // act: the (0,0) workgroup also takes ihelm's log-term step; else a launch of its
+  // own, after every read of ln for the (0,0) correction, does
   // algorithmic bytes: s, N and N_p's active rows in, the right-hand side out
   const double nzk = (double)k.nzdim - ((zhi >= zlo) ? (double)(zhi - zlo + 1) : 0.0);
-  ProbeScope probe(c, MLX_PROBE_ABCN_RHS, 64.0 * nzk * active_pairs(k, nroff, pcut), 0.0);
-  probed_launch(probe, k_abcn_rhs_d2_, grid, dim3(256), lds, c->stream, e, ln, nl, nlp, k.d2c, k.lognorm, k.ak,
+  ProbeScope probe(c, MLX_PROBE_ABCN_RHS, nf * 64.0 * nzk * active_pairs(k, nroff, pcut), 0.0);
+  probed_launch(probe, k_abcn_rhs_d2_, grid, dim3(256), lds, c->stream, f[0], f[nf - 1], k.d2c, k.lognorm, k.ak,
                 k.nrdim, k.npdim, k.ne, nrc, k.npchop, k.chopzl, k.chopzu, k.ell, dt, a, c->p.visc, pcut, zlo, zhi,
-                helm_pre ? nlln : nullptr, helm_pre ? nlpln : nullptr, helm_pre ? 1 : 0);
-  if (!helm_pre) hipLaunchKernelGGL(k_abcn_ln_, dim3(1), dim3(1), 0, c->stream, ln, ln, nlln, nlpln, dt, a);
+                act ? 1 : 0, keep ? 1 : 0);
+  if (!act)
+    for (int q = 0; q < nf; ++q)
+      hipLaunchKernelGGL(k_abcn_ln_pre_, dim3(1), dim3(1), 0, c->stream, f[q], k.lognorm, dt, a, k.ell,
+                         keep ? 1 : 0);
   HIPCHK(hipGetLastError());
 }
 
