@@ -637,8 +637,7 @@ void trans_adjoint_nolog_n(mlx_ctx *c, mlx_field *const *gs, int nf, bool to_fff
     // B^T = Z_b^T L_b^T Phi_b^T (L_b^T = L_f W^-1, Z_b^T = nz Z_f)
     for (int q = 0; q < nf; ++q) e[q] = gs[q]->e;
     fft_phi_batch(c, e, e, nf, -1);
-    for (int q = 0; q < nf; ++q)
-      k_adj_diag(c, gs[q]->e, -1, rmodes[q], k.np > 1 ? +1 : 0, k.nz > 1 ? (double)k.nz : 1.0);
+    k_adj_diag(c, gs, nf, -1, rmodes, k.np > 1 ? +1 : 0, k.nz > 1 ? (double)k.nz : 1.0);
     leg_n(c, gs, nf, false, nc, !lim);
     z(-1);
     for (int q = 0; q < nf; ++q) set_space(gs[q], "FFF");
@@ -646,8 +645,8 @@ void trans_adjoint_nolog_n(mlx_ctx *c, mlx_field *const *gs, int nf, bool to_fff
     // F^T = Phi_f^T L_f^T Z_f^T (L_f^T = W L_b, Z_f^T = Z_b / nz)
     z(+1);
     leg_n(c, gs, nf, true, nc, !lim);
+    k_adj_diag(c, gs, nf, +1, rmodes, k.np > 1 ? -1 : 0, k.nz > 1 ? 1.0 / k.nz : 1.0);
     for (int q = 0; q < nf; ++q) {
-      k_adj_diag(c, gs[q]->e, +1, rmodes[q], k.np > 1 ? -1 : 0, k.nz > 1 ? 1.0 / k.nz : 1.0);
       e[q] = gs[q]->e;
       set_space(gs[q], "PPP");
     }
@@ -810,8 +809,8 @@ void pff_adjoint_n(mlx_ctx *c, mlx_field *const *gs, int nf, const int *rmodes, 
       fft_z_batch(c, e, nf, +1, (double)k.nrdim * k.npdim);
   }
   double2 *e[kZBatch];
+  k_adj_diag(c, gs, nf, 0, rmodes, k.np > 1 ? -1 : 0, k.nz > 1 ? 1.0 / k.nz : 1.0);
   for (int q = 0; q < nf; ++q) {
-    k_adj_diag(c, gs[q]->e, 0, rmodes[q], k.np > 1 ? -1 : 0, k.nz > 1 ? 1.0 / k.nz : 1.0);
     e[q] = gs[q]->e;
     set_space(gs[q], "PPP");
   }

@@ -502,7 +502,7 @@ void k_adj_wscale(mlx_ctx *c, double2 *e, int mode);
 void k_ln_adjoint(mlx_ctx *c, const double2 *e, double *ln_bar, double sign);
 void k_adj_scale(mlx_ctx *c, double2 *e, double s);
 void k_adj_project(mlx_ctx *c, double2 *e);
-void k_adj_diag(mlx_ctx *c, double2 *e, int wmode, int rmode, int phimode, double s);
+void k_adj_diag(mlx_ctx *c, mlx_field *const *f, int nf, int wmode, const int *rmodes, int phimode, double s);
 void k_adj_sum_mask(mlx_ctx *c, double2 *sb, double *sbl, const double2 *g, const double *gl);
 void k_del2_t(mlx_ctx *c, double2 *out, const double2 *in, bool with_ak);
 void k_lap_ln_t(mlx_ctx *c, const double2 *e, double *ln_bar, double scale);
