@@ -442,6 +442,7 @@ void abcn(mlx_ctx *c, mlx_field *s, mlx_field *s_p, mlx_field *nl, mlx_field *nl
     MLX_THROW(MLX_E_ARG, "ihelm: alpha equals to zero. Inversion of 0*identity is impossible");
   // nl_p <- nl rides on the right-hand side where no field is given twice
   const bool keep = !lim && !swap_nl && nl_p != nl && nl_p != s && nl_p != s_p && nl != s && nl != s_p;
+  if (keep) k_helm_ready(c, a, 0, s->off[0]);  // a system that cannot be factored leaves s and nl_p as they are
   const AbcnRhs f = {s->e, s->sc, nl->e, nl->sc, nl_p->e, nl_p->sc};
   k_abcn_rhs_d2(c, &f, 1, dt, a, s->off[0], lim ? dl->pcut : -1, lim ? dl->zlo : 1, lim ? dl->zhi : 0, lim, keep);
   k_helm_solve(c, s->e, a, 0, s->off[0], lim ? dl->pcut : -1, lim ? dl->zlo : 1, lim ? dl->zhi : 0);

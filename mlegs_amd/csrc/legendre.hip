@@ -22,8 +22,8 @@
 // Every precision, FP64 included, takes the MFMA kernels of legendre_mfma.hip
 // and legendre_f64.hip where mfma_ok holds (same results bit for bit): at 256^3
 // the FP64 forward and backward contractions take 229 and 194 us here against
-// 122 and 106 us there, the projection 756 against 311 us with the de-aliasing
-// limits, and the default FP64 vortex step took 4.36 ms against 2.15.
+// 122 and 105 us there, the projection 756 against 282 us with the de-aliasing
+// limits, and the default FP64 vortex step took 4.36 ms against 2.11.
 #include "mlx_internal.h"
 
 namespace {

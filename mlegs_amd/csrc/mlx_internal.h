@@ -438,6 +438,8 @@ void k_zeroat1(mlx_ctx *c, double2 *e, int nrc, double2 *e2 = nullptr, int nrc2 
 void k_delsqp(mlx_ctx *c, double2 *e, double *ln, int nroff, int inverse);
 void k_bandmul(mlx_ctx *c, double2 *e, double *ln, int op, int nroff);  // op 0 del2, 1 del2h, 2 xxdx
 void k_helm_pre(mlx_ctx *c, double2 *e, double *ln_out, const double *ln_in, double alpha);
+// the factors of k_helm_solve(alpha, kind, nroff) now, if they are not kept
+void k_helm_ready(mlx_ctx *c, double alpha, int kind, int nroff);
 // pcut > 0: columns m >= pcut and kappa slices zlo..zhi are left unsolved
 // (for a caller that de-aliases the result)
 // e2 (optional): a second field solved with the same factors in the same launch

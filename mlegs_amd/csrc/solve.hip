@@ -624,6 +624,8 @@ LuCache &lu_get(mlx_ctx *c, double alpha, int kind, int nroff) {
 
 namespace mlx {
 
+void k_helm_ready(mlx_ctx *c, double alpha, int kind, int nroff) { (void)lu_get(c, alpha, kind, nroff); }
+
 void k_helm_solve(mlx_ctx *c, double2 *e, double alpha, int kind, int nroff, int pcut, int zlo, int zhi,
                   double2 *e2) {
   const KitDev &k = c->kit;
