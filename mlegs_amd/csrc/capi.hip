@@ -1054,7 +1054,7 @@ void vec2tp_pfp(mlx_ctx *c, mlx_field *ur, mlx_field *up, mlx_field *uz, mlx_fie
     // right-hand sides) are not visited
     to_fff(c, chi);
     k_helm_solve(c, chi->e, 0.0, 1, chi->off[0], dl.pcut, dl.zlo, dl.zhi);
-    k_idel2_post(c, chi->e, chi->sc);
+    if (!ln_zero) k_idel2_post(c, chi->e, chi->sc);
   } else {
     idel2_proln(c, chi);
   }
@@ -1136,15 +1136,17 @@ int advection_rhs(mlx_ctx *c, mlx_field *psi, mlx_field *chi, mlx_field *nlpsi, 
 // flag_dev (optional): the non-finite check of the field, on the same pass
 // dl (the time loop, right after de-aliasing f): the reduction skips the
 // de-aliased modes, which are zero
-// f2 (optional): a second field filtered in the same launches, gain gain2
+// f2 (optional): a second field filtered in the same launches, gain gain2;
+// zeroat: zeroat1 on the filtered fields, on the same pass
 void svv(mlx_ctx *c, mlx_field *f, double *gain_dev, int *flag_dev = nullptr, const DealiasLimits *dl = nullptr,
-         mlx_field *f2 = nullptr, double *gain2 = nullptr) {
+         mlx_field *f2 = nullptr, double *gain2 = nullptr, bool zeroat = false) {
   if (!c->p.is_svv) return;
   if (!is_fff(f) || (f2 && !is_fff(f2))) MLX_THROW(MLX_E_LAYOUT, "svv_filter: scalar must be in FFF space");
   need_kit(c);
   const bool lim = dl && dl->on;
+  const int zrc[2] = {c->kit.nrchop + f->off[0], c->kit.nrchop + (f2 ? f2 : f)->off[0]};
   k_svv(c, f->e, gain_dev, f2 ? f2->e : nullptr, gain2, flag_dev, lim ? dl->pcut : -1, lim ? dl->zlo : 1,
-        lim ? dl->zhi : 0);
+        lim ? dl->zhi : 0, nullptr, nullptr, zeroat ? zrc : nullptr);
 }
 
 void check_finite(mlx_ctx *c, const mlx_field *a, const mlx_field *b, int *flag_dev) {
@@ -1866,8 +1868,8 @@ void vortex_steps(mlx_ctx *c, mlx_vortex *v, int32_t nsteps, double dt, int32_t 
       // non-finite entries: the filter and zeroat1 keep a finite field
       // finite and a non-finite one non-finite, so the flag is the one the
       // check after the step would raise
-      svv(c, psi, v->gains, v->flag, &dl, chi, v->gains + 1);
-      zeroat1_pair(c, psi, chi);
+      if (c->p.is_svv) svv(c, psi, v->gains, v->flag, &dl, chi, v->gains + 1, true);
+      else zeroat1_pair(c, psi, chi);
       const int fmt = advection_rhs(c, psi, chi, nlpsi, nlchi, uz, true);
       if (!c->p.is_svv) check_finite(c, psi, chi, v->flag);
       // psi and chi are needed only where v and w are not kept

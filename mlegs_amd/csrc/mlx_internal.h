@@ -426,7 +426,8 @@ void k_dealias(mlx_ctx *c, double2 *e, const char *space);
 // field) in memory the caller provides instead of the context's
 constexpr int kSvvParts = 4096;
 void k_svv(mlx_ctx *c, double2 *e0, double *g0, double2 *e1 = nullptr, double *g1 = nullptr, int *flag = nullptr,
-           int pcut = -1, int zlo = 1, int zhi = 0, double *part_ws = nullptr, double *out_ws = nullptr);
+           int pcut = -1, int zlo = 1, int zhi = 0, double *part_ws = nullptr, double *out_ws = nullptr,
+           const int *zrc = nullptr);  // zrc: zeroat1 after it, rows of e0 and e1
 // noalloc.hip: looks up this device's static scratch array (once per device;
 // the device must be current)
 void noalloc_setup(int device);

@@ -180,25 +180,56 @@ __global__ void k_svv_gain(SvvFields F, const double *part, int nb, double *out,
   o[0] = fmin(strength0 * gn, 1.0);
 }
 
+// at1 given (the time loop): zeroat1 follows in the same launch.  The workgroups
+// blockIdx.x < nz filter column 0 of their slice and take its value at infinity
+// off, as k_zeroat1_ does (same sums in the same order); the others leave column 0.
 __global__ void k_svv_apply(SvvFields F, int nrdim, int npdim, int nz, double inv_r, double inv_p,
-                            const double *ak, double kmax, double cutoff, const double *out) {
+                            const double *ak, double kmax, double cutoff, const double *out, const double *at1,
+                            int zn0, int zn1) {
+  __shared__ double sh[16];
   const int f = blockIdx.y;
   const double st = out[3 * f];
-  if (!(st > 0.0)) return;
   double2 *e = F.e[f];
+  auto damp = [&](double q, double2 v) {
+    double s = (q - cutoff) / (1.0 - cutoff);
+    double s2 = s * s, s4 = s2 * s2;
+    double f2 = exp(-st * (s4 * s4));
+    return make_double2(f2 * v.x, f2 * v.y);
+  };
+  const int nzero = at1 ? nz : 0;
+  if ((int)blockIdx.x < nzero) {
+    const int k = blockIdx.x, n = f ? zn1 : zn0;
+    double2 *c = e + (size_t)k * nrdim * npdim;
+    double sr = 0.0, si = 0.0;
+    double2 v0 = make_double2(0.0, 0.0);
+    for (int i = threadIdx.x; i < nrdim; i += blockDim.x) {
+      const double q = svv_q(i, 0, k, inv_r, inv_p, ak, kmax);
+      double2 v = c[i];
+      if (st > 0.0 && q > cutoff) c[i] = v = damp(q, v);
+      if (i < n) {
+        sr += v.x * at1[i];
+        si += v.y * at1[i];
+      }
+      if (i == 0) v0 = v;
+    }
+    double a = block_sum(sr, sh);
+    double b = block_sum(si, sh);
+    if (threadIdx.x == 0) {
+      double d = at1[0];
+      c[0] = make_double2(v0.x - a / d, v0.y - b / d);
+    }
+    return;
+  }
+  if (!(st > 0.0)) return;
   size_t n = (size_t)nrdim * npdim * nz;
-  for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (size_t)gridDim.x * blockDim.x) {
+  const size_t stride = (size_t)(gridDim.x - nzero) * blockDim.x;
+  for (size_t t = (size_t)(blockIdx.x - nzero) * blockDim.x + threadIdx.x; t < n; t += stride) {
     int i = (int)(t % nrdim);
     int j = (int)((t / nrdim) % npdim);
     int k = (int)(t / ((size_t)nrdim * npdim));
+    if (at1 && j == 0) continue;
     double q = svv_q(i, j, k, inv_r, inv_p, ak, kmax);
-    if (q > cutoff) {
-      double s = (q - cutoff) / (1.0 - cutoff);
-      double s2 = s * s, s4 = s2 * s2;
-      double f2 = exp(-st * (s4 * s4));
-      double2 v = e[t];
-      e[t] = make_double2(f2 * v.x, f2 * v.y);
-    }
+    if (q > cutoff) e[t] = damp(q, e[t]);
   }
 }
 
@@ -1501,8 +1532,14 @@ void k_dealias(mlx_ctx *c, double2 *e, const char *space) {
                      pcut, zcut, zupper);
 }
 
+// rows of column 0 that zeroat1 sums, of a field with nrc rows
+static int zeroat1_rows(const KitDev &k, int nrc) {
+  const int n = nrc < k.nrchop ? nrc : k.nrchop;
+  return n > k.nrdim ? k.nrdim : n;
+}
+
 void k_svv(mlx_ctx *c, double2 *e0, double *g0, double2 *e1, double *g1, int *flag, int pcut, int zlo, int zhi,
-           double *part_ws, double *out_ws) {
+           double *part_ws, double *out_ws, const int *zrc) {
   const KitDev &k = c->kit;
   const mlx_params &p = c->p;
   double inv_r = 1.0 / fmax((double)(k.nrchop - 1), 1.0);
@@ -1529,8 +1566,9 @@ void k_svv(mlx_ctx *c, double2 *e0, double *g0, double2 *e1, double *g1, int *fl
                      inv_p, k.ak, kmax, cutoff, part, flag, ncol, zlo, zhi);
   hipLaunchKernelGGL(k_svv_gain, dim3(nf), dim3(1024), 0, c->stream, F, part, nbx * k.nzdim, out, target, relax,
                      st0);
-  hipLaunchKernelGGL(k_svv_apply, dim3(grid_for(c->nelem), nf), dim3(kT), 0, c->stream, F, k.nrdim, k.npdim,
-                     k.nzdim, inv_r, inv_p, k.ak, kmax, cutoff, out);
+  hipLaunchKernelGGL(k_svv_apply, dim3(grid_for(c->nelem) + (zrc ? k.nzdim : 0), nf), dim3(kT), 0, c->stream, F,
+                     k.nrdim, k.npdim, k.nzdim, inv_r, inv_p, k.ak, kmax, cutoff, out, zrc ? k.at1 : nullptr,
+                     zrc ? zeroat1_rows(k, zrc[0]) : 0, zrc && nf == 2 ? zeroat1_rows(k, zrc[1]) : 0);
 }
 
 void k_calcat(mlx_ctx *c, const double2 *e, const double *tbl, int nrc, double2 *out) {
@@ -1542,12 +1580,8 @@ void k_calcat(mlx_ctx *c, const double2 *e, const double *tbl, int nrc, double2 
 
 void k_zeroat1(mlx_ctx *c, double2 *e, int nrc, double2 *e2, int nrc2, double *lnz, double *lnz2) {
   const KitDev &k = c->kit;
-  auto rows = [&](int nrc_) {
-    int n = nrc_ < k.nrchop ? nrc_ : k.nrchop;
-    return n > k.nrdim ? k.nrdim : n;
-  };
   const int nf = e2 ? 2 : 1;
-  Zat1Fields F{{e, e2 ? e2 : e}, {rows(nrc), rows(e2 ? nrc2 : nrc)}, {lnz, e2 ? lnz2 : nullptr}};
+  Zat1Fields F{{e, e2 ? e2 : e}, {zeroat1_rows(k, nrc), zeroat1_rows(k, e2 ? nrc2 : nrc)}, {lnz, e2 ? lnz2 : nullptr}};
   hipLaunchKernelGGL(k_zeroat1_, dim3(k.nzdim, nf), dim3(kT), 0, c->stream, F, k.at1, k.nrdim, k.npdim);
 }
 
