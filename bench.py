@@ -16,12 +16,13 @@ Precisions (--prec) of the Legendre contractions; everything else is FP64:
          projection in FP32 except its m = 0 column in FP64 MFMA
   fp32   FP32 MFMA everywhere
   fp64m  FP64 MFMA everywhere
-  fp64   the plain FP64 path: FP64 vector-FMA contractions over every column,
-         no de-aliasing restrictions (the reference's operation set)
+  fp64   the library's default: FP64 MFMA too wherever its kernels cover the
+         grid (bit for bit the general FP64 kernels' results), with the
+         de-aliasing limits; fp64m asks for it by name
 
 Printed: one JSON line with
   value            steps/s of the selected precision
-  fp64_steps_per_s the same-GPU plain FP64 path over the same steps
+  fp64_steps_per_s the same-GPU FP64 path over the same steps
   gate             the accuracy gate of the metric: the selected precision's
                    psi and chi after a --traj-steps trajectory against the
                    plain FP64 path's, norm-wise relative, <= 1e-6
