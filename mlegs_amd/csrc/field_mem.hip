@@ -10,11 +10,13 @@
 // for the device covers the work of every stream that was issued before the
 // block was given up, the caller's own streams included; only then is it handed
 // out again.  32 blocks in limbo are enough for one such hipFree (of the
-// smallest of them).  What is kept is bounded per device (kMaxBytes, kMaxBlocks;
-// a block over kMaxBlock is freed at once), is returned when an allocation of
-// this library finds no memory, and when the device's last context ends.
-// Blocks are matched by size alone, under a mutex: no owner, stream or address
-// plays a part.
+// smallest of them).  A hipFree that fails (it is refused while any stream of the
+// process records a graph) has waited for nothing: its block and limbo stay as
+// they are until a later one succeeds.  What is kept is bounded per device
+// (kMaxBytes, kMaxBlocks; a block over kMaxBlock is freed at once), is returned
+// when an allocation of this library finds no memory, and when the device's last
+// context ends.  Blocks are matched by size alone, under a mutex: no owner,
+// stream or address plays a part.
 #include <mutex>
 
 #include "mlx_internal.h"
@@ -34,14 +36,21 @@ struct Pool {
   size_t bytes = 0;  // of both
   int contexts = 0;
 
-  void drop(Block b) {
-    (void)hipFree(b.p);
+  // whether b was freed, which is also whether the device has been waited for
+  bool drop(Block b) {
+    if (hipFree(b.p) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
     bytes -= b.bytes;
+    return true;
   }
   void release() {
     for (auto *v : {&limbo, &ready}) {
-      for (const Block &b : *v) drop(b);
-      v->clear();
+      size_t left = 0;
+      for (size_t i = 0; i < v->size(); ++i)
+        if (!drop((*v)[i])) (*v)[left++] = (*v)[i];
+      v->resize(left);
     }
   }
 };
@@ -77,18 +86,20 @@ void field_mem_put(int device, void *p, size_t bytes) {
   if (!p) return;
   std::lock_guard<std::mutex> lock(g_mutex);
   Pool &q = pools()[device];
-  if (q.contexts <= 0 || bytes > kMaxBlock || q.bytes + bytes > kMaxBytes || q.limbo.size() + q.ready.size() >= kMaxBlocks) {
-    (void)hipFree(p);
-  } else {
-    q.limbo.push_back({p, bytes});
-    q.bytes += bytes;
-    if (q.limbo.size() < kLimbo) return;
-    size_t least = 0;
-    for (size_t i = 1; i < q.limbo.size(); ++i)
-      if (q.limbo[i].bytes < q.limbo[least].bytes) least = i;
-    q.drop(q.limbo[least]);
-    q.limbo.erase(q.limbo.begin() + least);
+  q.limbo.push_back({p, bytes});
+  q.bytes += bytes;
+  if (q.contexts <= 0) {
+    q.release();
+    return;
   }
+  size_t out = q.limbo.size() - 1;  // the block to free: this one where it is not to be kept, else the smallest
+  if (bytes <= kMaxBlock && q.bytes <= kMaxBytes && q.limbo.size() + q.ready.size() <= kMaxBlocks) {
+    if (q.limbo.size() < kLimbo) return;
+    for (size_t i = 0; i < q.limbo.size(); ++i)
+      if (q.limbo[i].bytes < q.limbo[out].bytes) out = i;
+  }
+  if (!q.drop(q.limbo[out])) return;
+  q.limbo.erase(q.limbo.begin() + out);
   // the hipFree has waited for all work on the device
   q.ready.insert(q.ready.end(), q.limbo.begin(), q.limbo.end());
   q.limbo.clear();
@@ -97,9 +108,9 @@ void field_mem_put(int device, void *p, size_t bytes) {
 bool field_mem_release(int device) {
   std::lock_guard<std::mutex> lock(g_mutex);
   Pool &q = pools()[device];
-  const bool any = q.bytes > 0;
+  const size_t held = q.bytes;
   q.release();
-  return any;
+  return q.bytes < held;
 }
 
 void field_mem_contexts(int device, int d) {

@@ -190,7 +190,7 @@ struct mlx_ctx {
 namespace mlx {
 void *field_mem_get(int device, size_t bytes);  // nullptr: no memory
 void field_mem_put(int device, void *p, size_t bytes);
-bool field_mem_release(int device);             // whether anything was held
+bool field_mem_release(int device);             // whether anything was given back
 void field_mem_contexts(int device, int d);     // a context begins (+1), ends (-1)
 }  // namespace mlx
 
