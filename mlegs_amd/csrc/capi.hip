@@ -35,6 +35,8 @@ mlx_field *field_new(mlx_ctx *c) {
   const size_t ne = sizeof(double2) * c->nelem, ns = sizeof(double) * 8;
   const bool cap = capturing(c);
   mlx_field *f = new mlx_field();
+  f->bytes = ne;
+  f->device = c->device;
   if (cap) {
     if (hipMalloc(&f->e, ne) == hipSuccess && hipMalloc(&f->sc, ns) != hipSuccess) (void)hipFree(f->e);
   } else {
@@ -49,10 +51,10 @@ mlx_field *field_new(mlx_ctx *c) {
   return f;
 }
 
-void field_free(mlx_ctx *c, mlx_field *f) {
+void field_free(mlx_field *f) {
   if (!f) return;
-  field_mem_put(c->device, f->e, sizeof(double2) * c->nelem);
-  field_mem_put(c->device, f->sc, sizeof(double) * 8);
+  field_mem_put(f->device, f->e, f->bytes);
+  field_mem_put(f->device, f->sc, sizeof(double) * 8);
   delete f;
 }
 
@@ -80,6 +82,8 @@ void fcopy(mlx_ctx *c, mlx_field *d, const mlx_field *s) {
 void fmove(mlx_field *d, mlx_field *s) {
   std::swap(d->e, s->e);
   std::swap(d->sc, s->sc);
+  std::swap(d->bytes, s->bytes);
+  std::swap(d->device, s->device);
   std::memcpy(d->space, s->space, 4);
   std::memcpy(d->off, s->off, sizeof(d->off));
 }
@@ -1208,7 +1212,7 @@ int mlx_ctx_destroy(mlx_ctx *c) {
   if (!c) return MLX_OK;
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
-  for (mlx_field *f : c->pool) field_free(c, f);
+  for (mlx_field *f : c->pool) field_free(f);
   c->pool.clear();
   field_mem_contexts(c->device, -1);
   lu_cache_free(c);
@@ -1341,7 +1345,7 @@ int mlx_field_create(mlx_ctx *c, mlx_field **out) {
 int mlx_field_destroy(mlx_ctx *c, mlx_field *f) {
   return guarded(c, [&] {
     if (capturing(c)) HIPCHK(hipStreamSynchronize(c->stream));  // refused there
-    field_free(c, f);
+    field_free(f);
   });
 }
 
@@ -1780,7 +1784,7 @@ int mlx_vortex_create(mlx_ctx *c, const mlx_field *psi, const mlx_field *chi, co
       HIPCHK(hipMemsetAsync(v->gains, 0, sizeof(double) * 2, c->stream));
       HIPCHK(hipMemsetAsync(v->flag, 0, sizeof(int), c->stream));
     } catch (...) {
-      for (mlx_field *f : v->f) field_free(c, f);
+      for (mlx_field *f : v->f) field_free(f);
       delete v;
       throw;
     }
@@ -1792,7 +1796,7 @@ int mlx_vortex_destroy(mlx_ctx *c, mlx_vortex *v) {
   return guarded(c, [&] {
     if (!v) return;
     HIPCHK(hipStreamSynchronize(c->stream));
-    for (mlx_field *f : v->f) field_free(c, f);
+    for (mlx_field *f : v->f) field_free(f);
     if (v->gains) (void)hipFree(v->gains);
     if (v->flag) (void)hipFree(v->flag);
     delete v;
