@@ -13,10 +13,12 @@
 // smallest of them).  A hipFree that fails (it is refused while any stream of the
 // process records a graph) has waited for nothing: its block and limbo stay as
 // they are until a later one succeeds.  What is kept is bounded per device
-// (kMaxBytes, kMaxBlocks; a block over kMaxBlock is freed at once), is returned
-// when an allocation of this library finds no memory, and when the device's last
-// context ends.  Blocks are matched by size alone, under a mutex: no owner,
-// stream or address plays a part.
+// (kMaxBytes, kMaxBlocks; a block over kMaxBlock is freed at once; at a bound the
+// largest ready block of another size goes instead, so that a size no longer in
+// use does not hold the place), and is returned when an allocation of this
+// library finds no memory and when a context of the device ends: the memory of
+// a kit that is closed does not stay behind.  Blocks are matched by size alone,
+// under a mutex: no owner, stream or address plays a part.
 #include <mutex>
 
 #include "mlx_internal.h"
@@ -92,14 +94,24 @@ void field_mem_put(int device, void *p, size_t bytes) {
     q.release();
     return;
   }
-  size_t out = q.limbo.size() - 1;  // the block to free: this one where it is not to be kept, else the smallest
-  if (bytes <= kMaxBlock && q.bytes <= kMaxBytes && q.limbo.size() + q.ready.size() <= kMaxBlocks) {
+  // the block to free: this one where it is not to be kept, another size's in
+  // its place where that is enough, else the smallest of a full limbo
+  const size_t over_bytes = q.bytes > kMaxBytes ? q.bytes - kMaxBytes : 0;
+  const bool over = over_bytes > 0 || q.limbo.size() + q.ready.size() > kMaxBlocks;
+  std::vector<Block> *from = &q.limbo;
+  size_t out = q.limbo.size() - 1;
+  if (bytes <= kMaxBlock && over) {
+    size_t most = 0;
+    for (size_t i = 0; i < q.ready.size(); ++i)
+      if (q.ready[i].bytes != bytes && q.ready[i].bytes >= over_bytes && q.ready[i].bytes > most)
+        from = &q.ready, most = q.ready[out = i].bytes;
+  } else if (bytes <= kMaxBlock) {
     if (q.limbo.size() < kLimbo) return;
     for (size_t i = 0; i < q.limbo.size(); ++i)
       if (q.limbo[i].bytes < q.limbo[out].bytes) out = i;
   }
-  if (!q.drop(q.limbo[out])) return;
-  q.limbo.erase(q.limbo.begin() + out);
+  if (!q.drop((*from)[out])) return;
+  from->erase(from->begin() + out);
   // the hipFree has waited for all work on the device
   q.ready.insert(q.ready.end(), q.limbo.begin(), q.limbo.end());
   q.limbo.clear();
@@ -117,7 +129,7 @@ void field_mem_contexts(int device, int d) {
   std::lock_guard<std::mutex> lock(g_mutex);
   Pool &q = pools()[device];
   q.contexts += d;
-  if (q.contexts <= 0) q.release();
+  if (d < 0) q.release();
 }
 
 }  // namespace mlx

@@ -1,6 +1,7 @@
 """The bookkeeping of kept field memory (csrc/field_mem.hip) on the CPU, with
 hipMalloc and hipFree replaced: a block that was given up is handed out again
-only after a hipFree that succeeded, which is what waits for the device."""
+only after a hipFree that succeeded, which is what waits for the device; and
+what is kept is given back when a context ends and makes room for other sizes."""
 import os
 import subprocess
 
@@ -111,9 +112,35 @@ static int refused_release() {
   return 0;
 }
 
+// a context that ends gives back what is kept, also while another context of the device lives
+static int context_end() {
+  field_mem_contexts(0, 1);
+  field_mem_contexts(0, 1);
+  for (void *p : some(70, 4096)) field_mem_put(0, p, 4096);
+  CHECK(!live.empty());
+  field_mem_contexts(0, -1);
+  CHECK(live.empty());
+  return 0;
+}
+
+// kept blocks of a size that is no longer asked for make room for the size that is
+static int other_size() {
+  const size_t old = (size_t)64 << 20;  // 32 of them are all that is kept
+  field_mem_contexts(0, 1);
+  for (void *p : some(64, old)) field_mem_put(0, p, old);
+  for (int round = 0; round < 40; ++round)
+    for (void *p : some(20, 1 << 20)) field_mem_put(0, p, 1 << 20);
+  const int before = frees;
+  for (int round = 0; round < 40; ++round)
+    for (void *p : some(20, 1 << 20)) field_mem_put(0, p, 1 << 20);
+  CHECK(frees - before <= 40);  // 800 when each goes straight to hipFree
+  return 0;
+}
+
 int main(int, char **argv) {
   const struct { const char *name; int (*fn)(); } all[] = {
-      {"refused_limbo", refused_limbo}, {"refused_large", refused_large}, {"refused_release", refused_release}};
+      {"refused_limbo", refused_limbo}, {"refused_large", refused_large}, {"refused_release", refused_release},
+      {"context_end", context_end}, {"other_size", other_size}};
   for (auto &t : all)
     if (!std::strcmp(argv[1], t.name)) return t.fn();
   return 2;
@@ -135,7 +162,7 @@ def driver(tmp_path_factory):
     return str(exe)
 
 
-@pytest.mark.parametrize('case', ['refused_limbo', 'refused_large', 'refused_release'])
+@pytest.mark.parametrize('case', ['refused_limbo', 'refused_large', 'refused_release', 'context_end', 'other_size'])
 def test_field_mem(driver, case):
     r = subprocess.run([driver, case], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
