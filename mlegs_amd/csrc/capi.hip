@@ -527,9 +527,10 @@ int tp2vec_back(mlx_ctx *c, mlx_field *const *f, int nf, int ncols = -1, int zlo
   const bool lean = nc < k.npchop && k.np > 1;
   // physical rows only, on the MFMA path: the radial transform hands the
   // phi transform its FP32 even/odd sums (half the bytes of the FP64 rows,
-  // which the phi transform forms from them exactly)
+  // which the phi transform forms from them exactly); a line of pairs must fit a
+  // column (nr = 2 and 4 do not: whole rows there)
   const bool fp32 = mfma_ok(k, 0) && !mfma_fp64(c);
-  const bool pairs = lean && phys_rows && fp32;
+  const bool pairs = lean && phys_rows && fp32 && pair_stride(k) <= k.nrdim;
   double2 *e[kZBatch];
   for (int q = 0; q < nf; ++q) {
     e[q] = f[q]->e;

@@ -797,7 +797,7 @@ void leg_backward_mfma(mlx_ctx *c, const double2 *in, double2 *out, int ncols, b
 
 void leg_backward_pairs_f32(mlx_ctx *c, const double2 *in, float4 *pairs, int ncols) {
   const KitDev &k = c->kit;
-  if ((k.nr & 1) || pair_stride(k) > k.nrdim) MLX_THROW(MLX_E_ARG, "rtrans_backward: radial pairs need an even nr");
+  if ((k.nr & 1) || pair_stride(k) > k.nrdim) MLX_THROW(MLX_E_ARG, "rtrans_backward: a line of radial pairs exceeds a column");
   const int nyt = (k.nzdim + KT - 1) / KT;
   const int npc = (ncols > 0 && ncols < k.npchop) ? ncols : k.npchop;
   dim3 grid = xcd_grid(npc, nyt);
