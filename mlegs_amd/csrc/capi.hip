@@ -419,9 +419,10 @@ DealiasLimits dealias_limits(mlx_ctx *c) {
 
 // vec2tp's result is solved over the rows of chi's own radial offset.  The
 // MFMA projection forms the rows below nrchop - m only, so an FP64 result with
-// an offset takes the general projection, which forms the three rows past them.
+// an offset takes the general projection, which forms the three rows past them;
+// so does every precision's on the radial grids where all of them are FP64.
 bool general_projection(const mlx_ctx *c, const mlx_field *chi) {
-  return chi->off[0] != 0 && stage_precision(c, MLX_STAGE_PROJ) == MLX_PREC_FP64;
+  return chi->off[0] != 0 && (stage_precision(c, MLX_STAGE_PROJ) == MLX_PREC_FP64 || !mfma_small(c->kit));
 }
 
 // abcn (mlegs_scalar_ops.f90:1200-1262); copy_prev = false skips s_p <- s
