@@ -67,7 +67,8 @@ extern "C" {
 #define MLX_STAGE_UP    1    /* vec2tp's radial transforms of r u_phi (to
                                 FFF for its value at r = inf, and back)    */
 #define MLX_STAGE_PROJ  2    /* vec2tp's five projection contractions,
-                                columns m >= 1                              */
+                                columns m >= 1 (MLX_PREC_FP64: column 0 too,
+                                whatever MLX_STAGE_PROJ0 says)              */
 #define MLX_STAGE_PROJ0 3    /* the same for column m = 0, where idel2's
                                 kappa = 0 Laplacian systems amplify the
                                 contraction's rounding; a setting that

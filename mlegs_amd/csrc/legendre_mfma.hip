@@ -825,8 +825,9 @@ void leg_backward_pairs_f32(mlx_ctx *c, const double2 *in, float4 *pairs, int nc
 // ncols > 0: columns m >= ncols are zero; kappa slices zlo..zhi are zero
 // (zlo > zhi: none), for a caller that de-aliases the result.
 // prec_m0: precision of column m = 0 (an MFMA precision; -1: c->prec).  When
-// it differs from c->prec, column 0 runs as a launch of its own on the
-// context's second stream, concurrently with the other columns' launch.
+// it differs from c->prec (other than plain FP64, which column 0 follows),
+// column 0 runs as a launch of its own on the context's second stream,
+// concurrently with the other columns' launch.
 void vec2tp_project_mfma(mlx_ctx *c, const double2 *ur, const double2 *up, const double2 *uz, double2 *psi,
                          double2 *chi, int ncols, int zlo, int zhi, int prec_m0) {
   const KitDev &k = c->kit;
@@ -841,7 +842,8 @@ void vec2tp_project_mfma(mlx_ctx *c, const double2 *ur, const double2 *up, const
   // the projection has no split-BF16 kernel: BF16X3 runs it in FP32
   if (prec_m0 == MLX_PREC_BF16X3) prec_m0 = MLX_PREC_FP32;
   const int prec_rest = f64 ? MLX_PREC_FP64_MFMA : MLX_PREC_FP32;
-  if (!mfma_small(k)) prec_m0 = -1;  // FP64 throughout
+  // FP64 throughout: past 256 radial points, and where plain FP64 is set
+  if (!mfma_small(k) || c->prec == MLX_PREC_FP64) prec_m0 = -1;
   const bool split = prec_m0 >= 0 && prec_m0 != prec_rest;
   bool f64_0 = f64;
   if (split) {

@@ -3,7 +3,8 @@
 A radial chopping offset on chi, whose solve reads three rows past the chopped
 ones: past 256 radial points every precision forms them in FP64, against the
 oracle (test_gpu_parity's 1e-10; chi through its Laplacian, the projection's own
-product)."""
+product).  And the projection's own precision set to FP64 where the context's is
+lower: every column is formed in FP64."""
 import numpy as np
 import pytest
 
@@ -39,3 +40,26 @@ def test_offset_past_256_points(prec, monkeypatch):
     so.del2(ochi, okit)
     assert rel_err(chi.e, ochi.e) < 1e-10
     tfm.close()
+
+
+@pytest.mark.parametrize('cfg', ['C1', 'SMALL', 'ODD'])
+@pytest.mark.parametrize('ctx', ['FP32', 'BF16X3'])
+def test_fp64_projection_of_a_reduced_context(cfg, ctx):
+    """The projection and the transform before it set to FP64: the result of a
+    context in FP64, bit for bit, column 0 included."""
+    import mlegs_amd as M
+    print('fp64 projection', cfg, ctx, flush=True)
+    p = C.params(getattr(C, cfg))
+    out = []
+    for prec in ('FP64', ctx):
+        tfm = M.Kit(p, precision=getattr(M, 'PREC_' + prec))
+        if prec != 'FP64':
+            tfm.set_stage_precision(M.STAGE_UP, M.PREC_FP64)
+            tfm.set_stage_precision(M.STAGE_PROJ, M.PREC_FP64)
+        v = [M.Scalar(tfm).upload(C.physical(tfm.dims, p, 70 + i), space='PPP') for i in range(3)]
+        psi, chi = M.Scalar(tfm), M.Scalar(tfm)
+        M.vec2tp(*v, psi, chi, tfm)
+        out.append((psi.e, psi.ln, chi.e, chi.ln))
+        tfm.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
