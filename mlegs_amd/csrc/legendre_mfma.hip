@@ -703,10 +703,13 @@ void mfma_tables(mlx_ctx *c) {
     if (p) (void)hipFree(p);
     if (dev_malloc(&p, sizeof(*p) * n) != hipSuccess) MLX_THROW(MLX_E_ALLOC, "kit: table allocation failed");
   };
-  alloc(k.pfg32);
-  alloc(k.tVg32);
-  alloc(k.tDg32);
-  alloc(k.tTg32);
+  const bool f32 = mfma_small(k);  // else nothing reads the FP32 tables (270 MB at 512 x 256)
+  if (f32) {
+    alloc(k.pfg32);
+    alloc(k.tVg32);
+    alloc(k.tDg32);
+    alloc(k.tTg32);
+  }
   alloc(k.pfg64);
   alloc(k.tVg64);
   alloc(k.tDg64);
@@ -715,10 +718,12 @@ void mfma_tables(mlx_ctx *c) {
   auto relayout = [&](auto *dst, const double *src, int rows) {
     hipLaunchKernelGGL(k_tbl_pxa, dim3(nb), dim3(256), 0, c->stream, src, dst, k.nrh, rows, rows, AP, k.npchop);
   };
-  relayout(k.pfg32, k.pf, k.ne);
-  relayout(k.tVg32, k.tV, k.nt);
-  relayout(k.tDg32, k.tD, k.nt);
-  relayout(k.tTg32, k.tT, k.nt);
+  if (f32) {
+    relayout(k.pfg32, k.pf, k.ne);
+    relayout(k.tVg32, k.tV, k.nt);
+    relayout(k.tDg32, k.tD, k.nt);
+    relayout(k.tTg32, k.tT, k.nt);
+  }
   relayout(k.pfg64, k.pf, k.ne);
   relayout(k.tVg64, k.tV, k.nt);
   relayout(k.tDg64, k.tD, k.nt);
