@@ -268,7 +268,9 @@ __device__ __forceinline__ void fft_group_of(int type, int N, int ns, int til, c
     case 16 * 1 + 1:  // length 1
       for (int l = threadIdx.x; l < (1 << til); l += blockDim.x) st(0, l, ld(0, l));
       break;
-    default: fft_group<5, 1>(N, ns, til, tw, sg, ld, st); break;
+    default:  // (5, 1): groups_of makes no others
+      fft_group<5, 1>(N, ns, til, tw, sg, ld, st);
+      break;
   }
 }
 
@@ -889,6 +891,11 @@ bool launch_fft4(mlx_ctx *c, ProbeScope &ps, int N, dim3 grid_y, const FftFields
 #undef MLX_FFT4_
 }
 
+// the pairs of passes that fft_group_of has a kernel for
+constexpr bool pair_built(int r1, int r2) {
+  return r1 == 4 ? r2 <= 4 : (r1 == 2 || r1 == 3) && (r2 == 3 || r2 == 5);
+}
+
 // The groups of a plan: the two whose larger one is the smallest (the most
 // lines in flight: a group of NG elements is one thread's), or, where two
 // groups of at most 16 do not cover the length, pairs of passes in turn.  Rows
@@ -907,7 +914,10 @@ FftGroups groups_of(const FftPlan &pl, int nrow, int nwg) {
     g.ns[g.ng++] = ns;
     ns *= r1 * r2;
   };
-  auto size = [&](int p, int n) { return n < 1 || n > 2 ? 1 << 30 : pl.radix[p] * (n > 1 ? pl.radix[p + 1] : 1); };
+  auto size = [&](int p, int n) {
+    if (n < 1 || n > 2 || (n == 2 && !pair_built(pl.radix[p], pl.radix[p + 1]))) return 1 << 30;
+    return pl.radix[p] * (n > 1 ? pl.radix[p + 1] : 1);
+  };
   int cut = 0, best = 17;
   for (int p = 1; p < pl.npass; ++p) {
     const int m = std::max(size(0, p), size(p, pl.npass - p));
