@@ -29,6 +29,13 @@ void need_kit(mlx_ctx *c) {
   if (!c->kit.ready) MLX_THROW(MLX_E_ARG, "transformation kit is not initialized");
 }
 
+void field_free(mlx_field *f) {
+  if (!f) return;
+  field_mem_put(f->device, f->e, f->bytes);
+  field_mem_put(f->device, f->sc, sizeof(double) * 8);
+  delete f;
+}
+
 // Under capture nothing may be allocated or freed, a kept block no more than a
 // new one: hipMalloc and hipFree refuse there.
 mlx_field *field_new(mlx_ctx *c) {
@@ -47,15 +54,13 @@ mlx_field *field_new(mlx_ctx *c) {
     delete f;
     MLX_THROW(MLX_E_ALLOC, "scalar_init: device allocation failed");
   }
-  k_zero_field(c, f->e, f->sc);
+  try {
+    k_zero_field(c, f->e, f->sc);
+  } catch (...) {
+    field_free(f);
+    throw;
+  }
   return f;
-}
-
-void field_free(mlx_field *f) {
-  if (!f) return;
-  field_mem_put(f->device, f->e, f->bytes);
-  field_mem_put(f->device, f->sc, sizeof(double) * 8);
-  delete f;
 }
 
 void fmeta(mlx_field *d, const mlx_field *s) {

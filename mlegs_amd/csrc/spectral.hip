@@ -1771,12 +1771,22 @@ void k_write_field(mlx_ctx *c, double2 *dst, double v) {
   hipLaunchKernelGGL(k_write_field_, dim3(grid_for(c->nelem)), dim3(kT), 0, c->stream, dst, c->nelem, v);
 }
 
+// A launch over n entries that reports its own refusal, as a copy or a memset
+// does (hipGetLastError would also report an earlier, unrelated one).
+static void launch_checked(mlx_ctx *c, const void *kernel, size_t n, void **args) {
+  HIPCHK(hipLaunchKernel(kernel, dim3(grid_for(n)), dim3(kT), args, 0, c->stream));
+}
+
 void k_copy_field(mlx_ctx *c, double2 *dst, const double2 *src, double *dln, const double *sln) {
-  hipLaunchKernelGGL(k_copy_field_, dim3(grid_for(c->nelem)), dim3(kT), 0, c->stream, dst, src, c->nelem, dln, sln);
+  size_t n = c->nelem;
+  void *args[] = {&dst, &src, &n, &dln, &sln};
+  launch_checked(c, reinterpret_cast<const void *>(k_copy_field_), n, args);
 }
 
 void k_zero_field(mlx_ctx *c, double2 *dst, double *sc) {
-  hipLaunchKernelGGL(k_zero_field_, dim3(grid_for(c->nelem)), dim3(kT), 0, c->stream, dst, c->nelem, sc);
+  size_t n = c->nelem;
+  void *args[] = {&dst, &n, &sc};
+  launch_checked(c, reinterpret_cast<const void *>(k_zero_field_), n, args);
 }
 
 void k_abcn_rhs(mlx_ctx *c, double2 *sh, double *shln, const double2 *s, const double *sln, const double2 *nl,
