@@ -71,10 +71,11 @@ void fmeta(mlx_field *d, const mlx_field *s) {
 // deep copy (mlegs_scalar_init.f90:106-140): data and ln in one launch, where two
 // copies are two launches and more host time each (a 32 x 16 x 8 round trip of the
 // transforms 36.7 us with them, 32.6 without); at 256^3, where launches
-// do not count, the runtime's copy is 2 of 42 us faster
+// do not count, the runtime's copy is 2 of 42 us faster.  Between devices too the
+// runtime copies: a kernel would need peer access.
 void fcopy(mlx_ctx *c, mlx_field *d, const mlx_field *s) {
   if (d == s) return;
-  if (sizeof(double2) * c->nelem < ((size_t)64 << 20)) {
+  if (sizeof(double2) * c->nelem < ((size_t)64 << 20) && d->device == c->device && s->device == c->device) {
     k_copy_field(c, d->e, s->e, d->sc, s->sc);
   } else {
     HIPCHK(hipMemcpyAsync(d->e, s->e, sizeof(double2) * c->nelem, hipMemcpyDeviceToDevice, c->stream));
