@@ -37,18 +37,20 @@ void field_free(mlx_field *f) {
 }
 
 // Under capture nothing may be allocated or freed, a kept block no more than a
-// new one: hipMalloc and hipFree refuse there.
+// new one: hipMalloc and hipFree refuse there.  New memory lies on the current
+// device, so it is kept for that one, whatever the context's is.
 mlx_field *field_new(mlx_ctx *c) {
   const size_t ne = sizeof(double2) * c->nelem, ns = sizeof(double) * 8;
   const bool cap = capturing(c);
   mlx_field *f = new mlx_field();
   f->bytes = ne;
   f->device = c->device;
+  (void)hipGetDevice(&f->device);
   if (cap) {
     if (hipMalloc(&f->e, ne) == hipSuccess && hipMalloc(&f->sc, ns) != hipSuccess) (void)hipFree(f->e);
   } else {
-    f->e = static_cast<double2 *>(field_mem_get(c->device, ne));
-    if (f->e && !(f->sc = static_cast<double *>(field_mem_get(c->device, ns)))) field_mem_put(c->device, f->e, ne);
+    f->e = static_cast<double2 *>(field_mem_get(f->device, ne));
+    if (f->e && !(f->sc = static_cast<double *>(field_mem_get(f->device, ns)))) field_mem_put(f->device, f->e, ne);
   }
   if (!f->sc) {
     delete f;

@@ -80,8 +80,8 @@ struct KitDev {
 struct mlx_field {
   double2 *e = nullptr;   // nrdim*npdim*nzdim complex
   double *sc = nullptr;   // device scalars: sc[0] = ln
-  size_t bytes = 0;       // of e, and its device: of the context that made the field, which need
-  int device = 0;         // not be the one that ends it
+  size_t bytes = 0;       // of e: the context that ends the field need not be the one that made it
+  int device = 0;         // where e and sc lie
   char space[4] = {'P', 'P', 'P', 0};
   int off[3] = {0, 0, 0};
 };
