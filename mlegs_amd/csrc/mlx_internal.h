@@ -80,11 +80,14 @@ struct KitDev {
 struct mlx_field {
   double2 *e = nullptr;   // nrdim*npdim*nzdim complex
   double *sc = nullptr;   // device scalars: sc[0] = ln
-  size_t bytes = 0;       // of e: the context that ends the field need not be the one that made it
-  int device = 0;         // where e and sc lie
   char space[4] = {'P', 'P', 'P', 0};
   int off[3] = {0, 0, 0};
+  size_t bytes = 0;       // of e: the context that ends the field need not be the one that made it
+  int device = 0;         // where e and sc lie
 };
+// programs that map a field's device memory read e, sc and space at these places
+static_assert(offsetof(mlx_field, sc) == 8 && offsetof(mlx_field, space) == 16 && offsetof(mlx_field, off) == 20,
+              "mlx_field's first members");
 
 // cached LU factors of (del2 + alpha) per (m, |kappa|) system (layout in solve.hip)
 struct LuCache {
