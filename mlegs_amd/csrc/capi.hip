@@ -1224,6 +1224,7 @@ int mlx_ctx_destroy(mlx_ctx *c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   for (mlx_field *f : c->pool) field_free(f);
   c->pool.clear();
+  if (c->kit_bytes) field_mem_kits(c->device, c->kit_bytes, -1);
   field_mem_contexts(c->device, -1);
   lu_cache_free(c);
   hyp_cache_free(c);
@@ -1280,6 +1281,7 @@ int mlx_kit_init(mlx_ctx *c) {
     kit_build(c);
     const KitDev &k = c->kit;
     c->nelem = (size_t)k.nrdim * k.npdim * k.nzdim;
+    if (!c->kit_bytes) field_mem_kits(c->device, c->kit_bytes = sizeof(double2) * c->nelem, +1);
     // a buffer sized by an earlier kit is allocated again on first use
     if (c->v2t_part) {
       HIPCHK(hipStreamSynchronize(c->stream));

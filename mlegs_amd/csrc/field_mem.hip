@@ -16,9 +16,11 @@
 // (kMaxBytes, kMaxBlocks; a block over kMaxBlock is freed at once; at a bound the
 // largest ready block of another size goes instead, so that a size no longer in
 // use does not hold the place), and is returned when an allocation of this
-// library finds no memory and when a context of the device ends: the memory of
-// a kit that is closed does not stay behind.  Blocks are matched by size alone,
-// under a mutex: no owner, stream or address plays a part.
+// library finds no memory, when the last kit with fields of a block's size ends,
+// and when the device's last context does.  (Returning everything with any
+// context costs the first pass on the next kit of the same size its allocations:
+// 17.4 against 13.4 ms of a vortex step at 256^3.)  Blocks are matched by size
+// alone, under a mutex: no owner, stream or address plays a part.
 #include <mutex>
 
 #include "mlx_internal.h"
@@ -37,6 +39,7 @@ struct Pool {
   std::vector<Block> limbo, ready;
   size_t bytes = 0;  // of both
   int contexts = 0;
+  std::map<size_t, int> kits;  // by the size of their fields
 
   // whether b was freed, which is also whether the device has been waited for
   bool drop(Block b) {
@@ -47,11 +50,12 @@ struct Pool {
     bytes -= b.bytes;
     return true;
   }
-  void release() {
+  // frees the blocks of one size (0: all)
+  void release(size_t size = 0) {
     for (auto *v : {&limbo, &ready}) {
       size_t left = 0;
       for (size_t i = 0; i < v->size(); ++i)
-        if (!drop((*v)[i])) (*v)[left++] = (*v)[i];
+        if ((size && (*v)[i].bytes != size) || !drop((*v)[i])) (*v)[left++] = (*v)[i];
       v->resize(left);
     }
   }
@@ -129,7 +133,15 @@ void field_mem_contexts(int device, int d) {
   std::lock_guard<std::mutex> lock(g_mutex);
   Pool &q = pools()[device];
   q.contexts += d;
-  if (d < 0) q.release();
+  if (q.contexts <= 0) q.release();
+}
+
+void field_mem_kits(int device, size_t bytes, int d) {
+  std::lock_guard<std::mutex> lock(g_mutex);
+  Pool &q = pools()[device];
+  if ((q.kits[bytes] += d) > 0) return;
+  q.kits.erase(bytes);
+  q.release(bytes);
 }
 
 }  // namespace mlx

@@ -171,6 +171,7 @@ struct mlx_ctx {
   int stage_prec[MLX_STAGE_COUNT] = {-1, -1, -1, -1};
   std::string err;
   size_t nelem = 0;
+  size_t kit_bytes = 0;  // of a field, as told to field_mem_kits
   // scratch buffers of one field each, and small device scratch
   double2 *scr[2] = {nullptr, nullptr};
   double *dsmall = nullptr;     // 4096 doubles of reduction scratch
@@ -197,6 +198,7 @@ void *field_mem_get(int device, size_t bytes);  // nullptr: no memory
 void field_mem_put(int device, void *p, size_t bytes);
 bool field_mem_release(int device);             // whether anything was given back
 void field_mem_contexts(int device, int d);     // a context begins (+1), ends (-1)
+void field_mem_kits(int device, size_t bytes, int d);  // a kit with fields of that size begins, ends
 }  // namespace mlx
 
 // hipMalloc; kept field memory is returned first where there is none left

@@ -1,7 +1,8 @@
 """The bookkeeping of kept field memory (csrc/field_mem.hip) on the CPU, with
 hipMalloc and hipFree replaced: a block that was given up is handed out again
 only after a hipFree that succeeded, which is what waits for the device; and
-what is kept is given back when a context ends and makes room for other sizes."""
+what is kept is given back with the last kit of its size and makes room for other
+sizes."""
 import os
 import subprocess
 
@@ -40,6 +41,7 @@ void *field_mem_get(int device, size_t bytes);
 void field_mem_put(int device, void *p, size_t bytes);
 bool field_mem_release(int device);
 void field_mem_contexts(int device, int d);
+void field_mem_kits(int device, size_t bytes, int d);
 }
 using namespace mlx;
 
@@ -112,13 +114,23 @@ static int refused_release() {
   return 0;
 }
 
-// a context that ends gives back what is kept, also while another context of the device lives
-static int context_end() {
-  field_mem_contexts(0, 1);
-  field_mem_contexts(0, 1);
-  for (void *p : some(70, 4096)) field_mem_put(0, p, 4096);
-  CHECK(!live.empty());
+// the last kit with fields of a size gives that size back, also while other contexts of the device live
+static int kit_end() {
+  for (int i = 0; i < 3; ++i) field_mem_contexts(0, 1);
+  field_mem_kits(0, 4096, 1);
+  field_mem_kits(0, 4096, 1);
+  field_mem_kits(0, 8192, 1);
+  std::vector<void *> a = some(40, 4096), b = some(40, 8192);
+  for (int i = 0; i < 40; ++i) field_mem_put(0, a[i], 4096), field_mem_put(0, b[i], 8192);
+  const size_t all = live.size();
+  field_mem_kits(0, 4096, -1);
   field_mem_contexts(0, -1);
+  CHECK(live.size() == all);  // the other kit's fields may still take them
+  field_mem_kits(0, 4096, -1);
+  field_mem_contexts(0, -1);
+  for (void *p : a) CHECK(!live.count(p));
+  CHECK(!live.empty());
+  field_mem_kits(0, 8192, -1);
   CHECK(live.empty());
   return 0;
 }
@@ -140,7 +152,7 @@ static int other_size() {
 int main(int, char **argv) {
   const struct { const char *name; int (*fn)(); } all[] = {
       {"refused_limbo", refused_limbo}, {"refused_large", refused_large}, {"refused_release", refused_release},
-      {"context_end", context_end}, {"other_size", other_size}};
+      {"kit_end", kit_end}, {"other_size", other_size}};
   for (auto &t : all)
     if (!std::strcmp(argv[1], t.name)) return t.fn();
   return 2;
@@ -162,7 +174,7 @@ def driver(tmp_path_factory):
     return str(exe)
 
 
-@pytest.mark.parametrize('case', ['refused_limbo', 'refused_large', 'refused_release', 'context_end', 'other_size'])
+@pytest.mark.parametrize('case', ['refused_limbo', 'refused_large', 'refused_release', 'kit_end', 'other_size'])
 def test_field_mem(driver, case):
     r = subprocess.run([driver, case], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
