@@ -62,8 +62,6 @@ struct Mma<float> {
   __device__ static inline acc mma(pk a, pk b, acc c) { return op(a, b, c); }
   __device__ static inline acc zero() { return acc{0.f, 0.f, 0.f, 0.f}; }
   __device__ static inline vec vzero() { return make_float4(0.f, 0.f, 0.f, 0.f); }
-  // field column that A row i carries (accumulator element r of lane l is row 4(l/16)+r)
-  __device__ static inline int arow(int i) { return i; }
 };
 template <>
 struct Mma<Bf3> {
@@ -77,7 +75,6 @@ struct Mma<Bf3> {
   __device__ static inline acc zero() { return acc{0.f, 0.f, 0.f, 0.f}; }
   __device__ static inline vec vzero() { return make_float4(0.f, 0.f, 0.f, 0.f); }
   // the BF16 accumulator layout is the FP32 one (element r of lane l is row 4(l/16)+r)
-  __device__ static inline int arow(int i) { return i; }
   __device__ static inline short bits(__bf16 x) { return __builtin_bit_cast(short, x); }
   __device__ static inline pk prep(const stage *v) {
     pk o;
@@ -223,7 +220,7 @@ __global__ void __launch_bounds__(256) k_leg_fwd_mf(const double2 *__restrict__ 
         for (int t = 0; t < 4; ++t) {
           S v[M::NV];
 #pragma unroll
-          for (int j = 0; j < M::NV; ++j) v[j] = Bs[p][xr + j][16 * t + M::arow(lane % 16)];
+          for (int j = 0; j < M::NV; ++j) v[j] = Bs[p][xr + j][16 * t + lane % 16];
           fa[t] = M::prep(v);
         }
 #pragma unroll
@@ -333,7 +330,7 @@ __global__ void __launch_bounds__(256) k_leg_bwd_mf(const double2 *__restrict__ 
         for (int t = 0; t < 4; ++t) {
           S v[M::NV];
 #pragma unroll
-          for (int j = 0; j < M::NV; ++j) v[j] = Es[p][ar + j][16 * t + M::arow(lane % 16)];
+          for (int j = 0; j < M::NV; ++j) v[j] = Es[p][ar + j][16 * t + lane % 16];
           fa[t] = M::prep(v);
         }
 #pragma unroll
@@ -460,11 +457,11 @@ __global__ void __launch_bounds__(256) k_leg_bwd_mf(const double2 *__restrict__ 
 // computed: the three rows of the radial offset are chopped afterwards by
 // the reference.  Tables tg[m][p][x][a] (V, D, T).
 // ---------------------------------------------------------------------------
-template <typename T, int AT>
+template <int AT>
 __global__ void __launch_bounds__(256) k_v2t_mf(const double2 *__restrict__ ur, const double2 *__restrict__ up,
                                                 const double2 *__restrict__ uz, double2 *__restrict__ psi,
-                                                double2 *__restrict__ chi, const T *__restrict__ tgV,
-                                                const T *__restrict__ tgD, const T *__restrict__ tgT,
+                                                double2 *__restrict__ chi, const float *__restrict__ tgV,
+                                                const float *__restrict__ tgD, const float *__restrict__ tgT,
                                                  const double *__restrict__ ak, int nrdim, int npdim, int nz, int nr,
                                                  int nrh, int nrc0, int npc, int nzc, int nzcu, int nyt, int zlo,
                                                  int zhi, int mbeg, int mend, int tpitch) {
@@ -473,11 +470,11 @@ __global__ void __launch_bounds__(256) k_v2t_mf(const double2 *__restrict__ ur, 
   constexpr int AP = 4 * AT * 16;
   constexpr int APP = AP + 16;
   constexpr int KV = 8;   // contraction chunk for this kernel
-  typedef Mma<T> MM;
-  typedef typename MM::vec vec;
+  typedef Mma<float> MM;
+  typedef MM::vec vec;
   constexpr int VE = MM::VE;
-  __shared__ T X[5][KV][BJP];
-  __shared__ T Tb[3][KV][APP];
+  __shared__ float X[5][KV][BJP];
+  __shared__ float Tb[3][KV][APP];
   // both parities and every kappa tile of a column m on one XCD: the two
   // parity workgroups read the same input columns and write interleaved
   // rows of the same output lines, which then meet in that XCD's L2
@@ -503,7 +500,7 @@ __global__ void __launch_bounds__(256) k_v2t_mf(const double2 *__restrict__ ur, 
   const double2 *cz = uz + (size_t)nrdim * m;
   const size_t tb = ((size_t)m * 2 + p) * nrh * tpitch;
   const double seo = (p == 0) ? 1.0 : -1.0;
-  typename MM::acc aps[AT][4], ach[AT][4];
+  MM::acc aps[AT][4], ach[AT][4];
 #pragma unroll
   for (int s = 0; s < AT; ++s)
 #pragma unroll
@@ -541,11 +538,11 @@ __global__ void __launch_bounds__(256) k_v2t_mf(const double2 *__restrict__ ur, 
         const double2 x3 = make_double2(-kv * roe.y, kv * roe.x);           // i kv oe(ur)
         const double2 x4 = make_double2(mv * kv * peo.x, mv * kv * peo.y);  // m kv eo(up)
         const double2 x5 = make_double2(-zeo.x, -zeo.y);                    // -eo(uz)
-        X[0][fx][2 * fkl] = (T)x1.x; X[0][fx][2 * fkl + 1] = (T)x1.y;
-        X[1][fx][2 * fkl] = (T)x2.x; X[1][fx][2 * fkl + 1] = (T)x2.y;
-        X[2][fx][2 * fkl] = (T)x3.x; X[2][fx][2 * fkl + 1] = (T)x3.y;
-        X[3][fx][2 * fkl] = (T)x4.x; X[3][fx][2 * fkl + 1] = (T)x4.y;
-        X[4][fx][2 * fkl] = (T)x5.x; X[4][fx][2 * fkl + 1] = (T)x5.y;
+        X[0][fx][2 * fkl] = (float)x1.x; X[0][fx][2 * fkl + 1] = (float)x1.y;
+        X[1][fx][2 * fkl] = (float)x2.x; X[1][fx][2 * fkl + 1] = (float)x2.y;
+        X[2][fx][2 * fkl] = (float)x3.x; X[2][fx][2 * fkl + 1] = (float)x3.y;
+        X[3][fx][2 * fkl] = (float)x4.x; X[3][fx][2 * fkl + 1] = (float)x4.y;
+        X[4][fx][2 * fkl] = (float)x5.x; X[4][fx][2 * fkl + 1] = (float)x5.y;
         __syncthreads();
       }
       const int xn = x0 + KV;  // chunk fetched now, stored next iteration
@@ -557,7 +554,7 @@ __global__ void __launch_bounds__(256) k_v2t_mf(const double2 *__restrict__ ur, 
           if (idx < 3 * KV * (AP / VE)) {
             const int a = VE * (idx % (AP / VE)), x = (idx / (AP / VE)) % KV, q = idx / ((AP / VE) * KV);
             const int xg = xn + x;
-            const T *src = (q == 0) ? tgV : (q == 1) ? tgD : tgT;
+            const float *src = (q == 0) ? tgV : (q == 1) ? tgD : tgT;
             if (xg < nrh) v = *reinterpret_cast<const vec *>(src + tb + (size_t)xg * tpitch + a);
           }
           rt[j] = v;
@@ -581,19 +578,19 @@ __global__ void __launch_bounds__(256) k_v2t_mf(const double2 *__restrict__ ur, 
   #pragma unroll
       for (int kk = 0; kk < KV; kk += 4) {
         const int xr = kk + lane / 16;
-        T f[5][4];
+        float f[5][4];
   #pragma unroll
         for (int q = 0; q < 5; ++q)
   #pragma unroll
-          for (int t = 0; t < 4; ++t) f[q][t] = X[q][xr][16 * t + MM::arow(lane % 16)];
+          for (int t = 0; t < 4; ++t) f[q][t] = X[q][xr][16 * t + lane % 16];
   #pragma unroll
         for (int s = 0; s < AT; ++s) {
           const int at = wv + 4 * s;
           if (at * 16 >= M) continue;
           const int al = (wv + 4 * s) * 16 + lane % 16;  // local table column
-          T bv = Tb[0][xr][al];
-          T bd = Tb[1][xr][al];
-          T bt = Tb[2][xr][al];
+          float bv = Tb[0][xr][al];
+          float bd = Tb[1][xr][al];
+          float bt = Tb[2][xr][al];
   #pragma unroll
           for (int t = 0; t < 4; ++t) {
             aps[s][t] = MM::op(f[0][t], bv, aps[s][t]);
@@ -867,7 +864,7 @@ void vec2tp_project_mfma(mlx_ctx *c, const double2 *ur, const double2 *up, const
     }
     dim3 grid = xcd_grid(me - mb, 2 * nyt);
 #define MLX_V2T(AT_)                                                                                                \
-  hipLaunchKernelGGL((k_v2t_mf<float, AT_>), grid, dim3(256), 0, s, ur, up, uz, psi, chi, k.tVg32, k.tDg32, k.tTg32, \
+  hipLaunchKernelGGL((k_v2t_mf<AT_>), grid, dim3(256), 0, s, ur, up, uz, psi, chi, k.tVg32, k.tDg32, k.tTg32, \
                      k.ak, k.nrdim, k.npdim, k.nzdim, k.nr, k.nrh, k.nrchop, npc, k.chopzl, k.chopzu, nyt, zlo, zhi, \
                      mb, me, k.mfma_ap)
     if (at == 1) MLX_V2T(1);
