@@ -148,7 +148,10 @@ int mlx_set_stage_precision(mlx_ctx* ctx, int stage, int prec);
 /* Allocate a scalar of the kit's global size, space "PPP", ln = 0, offsets 0.
  * Replaces scalar%init (src/submodules/mlegs_scalar_init.f90:6-67). */
 int mlx_field_create(mlx_ctx* ctx, mlx_field** out);
-/* scalar%dealloc (src/submodules/mlegs_scalar_init.f90:70-81). */
+/* scalar%dealloc (src/submodules/mlegs_scalar_init.f90:70-81).  Does not
+ * wait for the stream: the field's memory is kept, at most 2 GiB per device,
+ * and goes to a later field once the device has finished what was issued
+ * before.  Refused while the context's stream records a graph. */
 int mlx_field_destroy(mlx_ctx* ctx, mlx_field* f);
 /* Deep copy dst = src: data, ln, offsets, space
  * (src/submodules/mlegs_scalar_init.f90:106-140). */

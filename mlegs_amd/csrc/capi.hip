@@ -1099,7 +1099,8 @@ void vec2tp(mlx_ctx *c, const mlx_field *vr, const mlx_field *vp, const mlx_fiel
 // already de-aliased (the stepper de-aliases them before svv_filter and
 // zeroat1, which keep a zero mode zero), so the opening dealias is a no-op.
 // Returns how v and w (v without the background flow) are left in the
-// temporaries 4..9: 2 in FP32, 1 in FP64, 0 not at all (overwritten).
+// temporaries 4..9: 2 in FP32, 1 in FP64, 0 where they are not FP64 values (formed
+// from FP32 sums) or not there at all (overwritten).
 int advection_rhs(mlx_ctx *c, mlx_field *psi, mlx_field *chi, mlx_field *nlpsi, mlx_field *nlchi,
                   const mlx_field *uz, bool dealiased = false) {
   if (!is_fff(psi) || !is_fff(chi)) MLX_THROW(MLX_E_LAYOUT, "advection_rhs: psi and chi must be in FFF");
@@ -1858,7 +1859,7 @@ int mlx_vortex_bootstrap(mlx_ctx *c, mlx_vortex *v) {
 // vortical_flow_3d.f90:160-181.  rec (optional): 2 nsteps fields that
 // receive psi and chi after each step; rec_vw (optional): 6 nsteps fields
 // that receive v (without the background flow) and w at them, where the
-// step leaves them (*vw_fmt: 2 FP32, 1 FP64, 0 not recorded)
+// step leaves them (*vw_fmt: 2 FP32, 1 FP64, 0 not recorded: advection_rhs's 0)
 void vortex_steps(mlx_ctx *c, mlx_vortex *v, int32_t nsteps, double dt, int32_t check, mlx_field **rec,
                   mlx_field **rec_vw = nullptr, int *vw_fmt = nullptr) {
   {

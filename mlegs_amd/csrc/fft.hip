@@ -12,9 +12,9 @@
 //
 // Design: one workgroup owns TI consecutive radial rows i of one (k) plane
 // (phi) or one (j) column (z), the line index fastest (coalesced global
-// access, conflict-free LDS).  Power-of-two lengths take the four-step kernels
-// (k_fft4, k_fft4_cross), the others the grouped Stockham kernels (k_fftg,
-// k_fftg_cross); both read a line element from HBM once, straight into
+// access, conflict-free LDS).  The powers of two from 16 to 256 take the
+// four-step kernels (k_fft4, k_fft4_cross), other lengths the grouped Stockham
+// kernels (k_fftg, k_fftg_cross); both read a line element from HBM once, straight into
 // registers, and write it once.  The real-to-complex phi transform is a
 // complex FFT of length np/2 plus the even/odd untangling step.  HBM-bound for
 // large fields, launch-bound for small ones: up to kZBatch fields share a launch.
@@ -99,7 +99,7 @@ __device__ inline void dft<5>(double2 *v, double sg) {
 }
 
 // ---------------------------------------------------------------------------
-// Fast path for power-of-two lengths N = N1 * N2 (N1, N2 <= 16): four-step
+// Fast path for the lengths N = N1 * N2 = 16 to 256 (powers of two): four-step
 // FFT.  Stage 1 loads x[n2 + N2 n1] of a line straight into registers, runs
 // the N1-point DFT over n1 there and applies W_N^{n2 k1}; one LDS exchange;
 // stage 2 runs the N2-point DFT over n2 and writes X[k1 + N1 k2].  A

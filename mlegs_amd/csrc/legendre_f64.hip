@@ -5,8 +5,8 @@
 // Both are GEMMs whose A operand is the field (16 rows = the real and
 // imaginary parts of 8 axial slices; element r of lane l of the accumulator is
 // row l/16 + 4r, measured on gfx950, so A row i carries field column 4(i%4) +
-// i/4 and that element is column 4(l/16) + r) and whose B operand is the table (16 radial rows or points).  A workgroup of 8 waves
-// takes KT slices of one column m.
+// i/4 and that element is column 4(l/16) + r) and whose B operand is the table (16
+// radial rows or points).  A workgroup of 8 waves takes KT slices of one column m.
 //
 // What bounds them: the FP64 MFMA (3.25 GFLOP, 45 us at the 72.6 TFLOP/s of a
 // large product) and the field's two passes over HBM (240-270 MB, about 50 us)
@@ -21,8 +21,9 @@
 //    staging by itself took 72 us of a 256^3 launch, now 32).
 //  - Output rows of both parities are put together in LDS and written as whole
 //    columns, streaming.
-// At 256^3, every column: forward 170 -> 122 us, backward 129 -> 106 us
-// (kernels that stage the table in LDS, one wave per SIMD, before).
+// At 256^3, every column, in the first nine round trips of a field: forward 170 ->
+// 122 us, backward 129 -> 105 us (kernels that stage the table in LDS, one wave per
+// SIMD, before); 116 and 101 over 33 round trips.
 #include "mlx_internal.h"
 
 namespace {
@@ -222,8 +223,8 @@ __global__ void __launch_bounds__(512) k_leg_fwd_f64m(LegFields f, LegDims d, co
 // backward: f(x) = be + bo, f(-x) = be - bo, b_p(x, k) = sum_a P(x, 2a+p)
 // e(2a+p, k), table ptab[m][n][x].  A wave owns 16 points x, both parities;
 // the workgroup the 128 points from 128 sp on.  KT = 16 and chunks of 8 for
-// every size (32 slices: 97 us at 256^3 against 96, and 10.4 against 7.9 at
-// 128 x 64 x 64).  f.ln: column 0 of the output plus ln lnx(x).
+// every size: one kernel (32 slices take 90 us at 256^3 against 97, but 13.1
+// against 11.4 at 128 x 64 x 64; round trips of one field).  f.ln: column 0 of the output plus ln lnx(x).
 __global__ void __launch_bounds__(512) k_leg_bwd_f64m(LegFields f, LegDims d, const double *__restrict__ ptab) {
   constexpr int KT = 16, AC = 8, NT = KT / 8, PC = 2 * KT + 2, KS = AC / 4;
   // the even and odd rows' planes: 64 bytes apart modulo the banks
@@ -340,8 +341,9 @@ struct V2tArgs {
 // Four waves (32 rows a, both parities) and 8 slices a workgroup for every size, held
 // to the registers of four workgroups a CU: at 256^3 282 us, where eight waves and
 // 32 slices (half the table and field reads from L2, one workgroup to a CU) take
-// 316, 16 slices 321, and this tile without the bound 320.  150 x 120 x 90: 51 us
-// against 76 with eight waves; one slice, 256 x 256: 25 against 37 with 16 slices.
+// 316, 16 slices 321, and this tile without the bound 316.  150 x 120 x 90: 45 us
+// (51 without the bound) against 76 with eight waves; one slice, 256 x 256: 25
+// against 37 with 16 slices.
 template <bool COL0>
 __global__ void __launch_bounds__(256, 4) k_v2t_f64m(V2tArgs g) {
   constexpr int NW = 4, KT = 8, NTH = 64 * NW, NT = KT / 8, XC = 8, KS = XC / 4, PC = 2 * KT + 2, PL = XC * PC, NB = 6 * PL;
@@ -526,8 +528,9 @@ void leg_forward_f64(mlx_ctx *c, const double2 *const *in, double2 *const *out, 
   const int M = (k.nrchop + 1) / 2;
   ProbeScope probe(c, MLX_PROBE_LEG_FWD, nf * leg_bytes(k, 0, 8, npc), nf * leg_flops(k, 0, npc));
   // 32 slices and 128 rows a workgroup where that still leaves two workgroups
-  // to a CU; 16 slices and 64 rows below (256^3: 101 us against 118; 128 x 64
-  // x 64, 66 workgroups of the large kind: 12.4 against 7.4 us)
+  // to a CU; 16 slices and 64 rows below (round trips of one field: at 256^3 112 us
+  // against 123 in the small tiles; at 128 x 64 x 64, 66 workgroups of the large
+  // kind, 17.4 against 11.0)
   const LegDims big = leg_dims(k, nf, npc, ncol, 32, (M + 127) / 128);
   const bool inplace = in[0] == out[0];
   if (inplace && !leg_inplace_ok(k)) MLX_THROW(MLX_E_ARG, "rtrans_forward: in place past 256 radial points");

@@ -680,9 +680,9 @@ int mfma_tiles(const KitDev &k) {
   return (M + 63) / 64;
 }
 
-// The largest radial grid of the MFMA kernels: that of the banded solves (544
-// rows).  Above 256 points they run in FP64 whatever the precision (as the
-// general kernels, which such kits took before, do).
+// The largest radial grid of the MFMA kernels: 640 points (the first whole groups
+// past the banded solves' 544 rows).  Above 256 points they run in FP64 whatever
+// the precision, as the general kernels do.
 constexpr int kMfmaGroups = 5;
 bool mfma_ok(const KitDev &k, int nroff) {
   const int at = mfma_tiles(k);
